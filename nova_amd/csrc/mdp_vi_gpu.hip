@@ -16,6 +16,7 @@
 //     reference's tie rule, and V'/pi are written coalesced.
 // A plain one-thread-per-state kernel covers shapes the tiled kernel does not (ns > 256,
 // m > 2048, misaligned arrays).
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <vector>
@@ -682,6 +683,128 @@ void vi_chunk_rows(unsigned n, unsigned m,
     }
 }
 
+// ---- small models: every sweep of a run in one launch
+//
+// At a few hundred states a sweep is bound by its launch and by the chain of loads behind it,
+// not by its bytes. A model whose (s, a, i) entries fit one workgroup's LDS is loaded there once
+// (the successor as 16 bits, gamma * T and R as floats, action-major so that lanes of
+// neighbouring states read neighbouring words) beside both value buffers, and one 1,024-lane
+// workgroup runs all sweeps of the run: P adjacent lanes per state (P a power of two, as many
+// as the lanes and actions allow) take every P-th action each, sum its row in the reference's
+// order, and merge by (value, lower action). One barrier per sweep. Products, sums and ties are
+// those of the other sweeps, so V and pi are the same bit for bit; both of the last two
+// iterates are written, as the ping-pong of separate sweeps leaves them. us per sweep, this
+// kernel against a graph of single sweeps in 128-row tiles: n = 100, m = ns = 4: 1.0 / 3.6;
+// n = 900, m = ns = 5: 3.3 / 5.4 (its 4,500 row chains and random LDS reads of one CU bound it).
+constexpr unsigned kResThreads = 1024;
+constexpr size_t kResLds = 160 * 1024;
+constexpr unsigned short kResEnd = 0xFFFF;   // past the row's end (so n <= 65,535)
+
+size_t resident_lds(size_t n, size_t m, size_t ns)
+{
+    const size_t rows = n * m;
+    return 4 * (2 * n + rows + rows * ns) + (2 * rows * ns + 3) / 4 * 4;
+}
+
+// EB: entries of a row requested together (a row takes ceil(ns / EB) rounds)
+template <unsigned EB>
+__global__ __launch_bounds__(kResThreads) void vi_resident(unsigned n, unsigned m, unsigned ns,
+        unsigned P, float gamma, const int *__restrict__ S, const float *__restrict__ T,
+        const float *__restrict__ R, const float *V0, float *Vlast, float *Vprev,
+        unsigned *__restrict__ pi, unsigned sweeps)
+{
+    extern __shared__ float smem[];
+    const unsigned rows = n * m, t = threadIdx.x;
+    float *Va = smem, *Vb = smem + n;
+    float *Rl = smem + 2 * n;                    // [a][s]
+    float *Tl = Rl + rows;                       // [i][a][s], times gamma
+    unsigned short *Sl = reinterpret_cast<unsigned short *>(Tl + rows * ns);
+    for (unsigned x = t; x < rows * ns; x += kResThreads) {
+        const unsigned row = x / ns, i = x % ns, s = row / m, a = row % m;
+        const int sp = S[x];
+        Sl[i * rows + a * n + s] = sp < 0 ? kResEnd : (unsigned short)min((unsigned)sp, n - 1);
+        Tl[i * rows + a * n + s] = __fmul_rn(gamma, T[x]);
+    }
+    for (unsigned row = t; row < rows; row += kResThreads)
+        Rl[(row % m) * n + row / m] = R[row];
+    for (unsigned s = t; s < n; s += kResThreads)
+        Va[s] = V0[s];
+    __syncthreads();
+    // entries after a row's first negative successor are ignored, whatever they hold
+    for (unsigned row = t; row < rows; row += kResThreads) {
+        bool end = false;
+        for (unsigned i = 0; i < ns; i++) {
+            end = end || Sl[i * rows + row] == kResEnd;
+            if (end)
+                Sl[i * rows + row] = kResEnd;
+        }
+    }
+    __syncthreads();
+    const unsigned p = t % P, step = kResThreads / P;
+    for (unsigned k = 0; k < sweeps; k++) {
+        const bool last = k + 1 == sweeps;
+        // every lane of a state's group makes the same trips (the merge reads all of them)
+        for (unsigned s = t / P; s < n; s += step) {
+            float best = -INFINITY, q0 = 0.0f;
+            unsigned bestA = 0xFFFFFFFFu;
+            for (unsigned a = p; a < m; a += P) {
+                const unsigned row = a * n + s;
+                float q = Rl[row];
+                for (unsigned i0 = 0; i0 < ns; i0 += EB) {
+                    unsigned short sp[EB];
+                    float g[EB];
+#pragma unroll
+                    for (unsigned i = 0; i < EB; i++) {
+                        const unsigned at = min(i0 + i, ns - 1) * rows + row;
+                        sp[i] = i0 + i < ns ? Sl[at] : kResEnd;
+                        g[i] = Tl[at];
+                    }
+#pragma unroll
+                    for (unsigned i = 0; i < EB; i++)
+                        g[i] = __fmul_rn(g[i], Va[sp[i] == kResEnd ? 0u : (unsigned)sp[i]]);
+#pragma unroll
+                    for (unsigned i = 0; i < EB; i++)
+                        q = sp[i] == kResEnd ? q : __fadd_rn(q, g[i]);
+                }
+                if (a == 0)
+                    q0 = q;
+                // action 0 is taken as it is, a later one only when strictly larger (so a NaN
+                // never beats anything, and a NaN at action 0 stays)
+                if (a == 0 || q > best || (q == best && bestA == 0xFFFFFFFFu)) {
+                    best = q;
+                    bestA = a;
+                }
+            }
+            for (unsigned off = 1; off < P; off <<= 1) {
+                const float ob = __shfl_xor(best, (int)off);
+                const unsigned oa = __shfl_xor(bestA, (int)off);
+                if (oa != 0xFFFFFFFFu &&
+                        (bestA == 0xFFFFFFFFu || ob > best || (ob == best && oa < bestA))) {
+                    best = ob;
+                    bestA = oa;
+                }
+            }
+            if (p == 0) {
+                if (q0 != q0) {
+                    best = q0;
+                    bestA = 0;
+                }
+                Vb[s] = best;
+                if (last)
+                    pi[s] = bestA;
+            }
+        }
+        __syncthreads();
+        float *sw = Va;
+        Va = Vb;
+        Vb = sw;
+    }
+    for (unsigned s = t; s < n; s += kResThreads) {
+        Vlast[s] = Va[s];
+        Vprev[s] = Vb[s];
+    }
+}
+
 // ---- batched value iteration: many MDPs of uneven size, one launch per sweep for all
 //
 // Every sweep of every instance is captured into one HIP graph: launch k runs sweep k of all
@@ -768,6 +891,25 @@ unsigned pow2_at_least(unsigned x)
 }
 
 } // namespace
+
+typedef void (*ResidentFn)(unsigned, unsigned, unsigned, unsigned, float, const int *,
+                           const float *, const float *, const float *, float *, float *,
+                           unsigned *, unsigned);
+
+static ResidentFn resident_for(unsigned ns)
+{
+    const unsigned rounds = (ns + 7) / 8;
+    switch ((ns + rounds - 1) / rounds) {
+    case 1: return vi_resident<1>;
+    case 2: return vi_resident<2>;
+    case 3: return vi_resident<3>;
+    case 4: return vi_resident<4>;
+    case 5: return vi_resident<5>;
+    case 6: return vi_resident<6>;
+    case 7: return vi_resident<7>;
+    default: return vi_resident<8>;
+    }
+}
 
 // Every sweep layout built gets a serial number of its own. The cached sweep graph is keyed by
 // it (not by the layout's address, which a later layout of other settings may reuse) and is
@@ -1281,11 +1423,49 @@ static void vi_graph_forget_layout(unsigned long long serial)
     }
 }
 
+// Whether a run of sweeps takes vi_resident: the model fits one workgroup's LDS and the run has
+// at least two sweeps (a single sweep gains nothing from loading the model first).
+// NOVA_AMD_VI_KERNEL=tiled keeps the launch per sweep.
+static bool resident_wanted(const ViPlan &plan, const nova::MDP *mdp, unsigned sweeps)
+{
+    if (plan.chunked || plan.sorted || sweeps < 2 || mdp->n > 65534u || mdp->m > kResLds ||
+            mdp->ns > kResLds || resident_lds(mdp->n, mdp->m, mdp->ns) > kResLds)
+        return false;
+    const char *f = std::getenv("NOVA_AMD_VI_KERNEL");
+    return f == nullptr || std::strcmp(f, "tiled") != 0;
+}
+
 static int vi_run_sweeps(const nova::MDP *mdp, nova::MDPVIGPU *vi, unsigned sweeps,
                          hipStream_t st, hipEvent_t t0, hipEvent_t t1, const char *fn)
 {
     const ViPlan plan = vi_plan(mdp, vi);
     const unsigned parity = vi->currentHorizon % 2;
+    if (resident_wanted(plan, mdp, sweeps)) {
+        const unsigned n = mdp->n, m = mdp->m;
+        const bool endEven = (parity + sweeps) % 2 == 0;
+        unsigned P = 1;
+        while (2 * P <= std::min(m, 64u) && (size_t)n * 2 * P <= kResThreads)
+            P *= 2;
+        const ResidentFn f = resident_for(mdp->ns);
+        hipFuncSetAttribute((const void *)f, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)kResLds);
+        if (t0) hipEventRecord(t0, st);
+        hipLaunchKernelGGL(f, dim3(1), dim3(kResThreads), resident_lds(n, m, mdp->ns), st, n, m,
+                           mdp->ns, P, mdp->gamma, mdp->d_S, mdp->d_T, mdp->d_R,
+                           parity == 0 ? vi->d_V : vi->d_VPrime,
+                           endEven ? vi->d_V : vi->d_VPrime, endEven ? vi->d_VPrime : vi->d_V,
+                           vi->d_pi, sweeps);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess)
+            return hip_fail(e, fn, "Failed to execute the sweeps.", NOVA_ERROR_KERNEL_EXECUTION);
+        if (t1) hipEventRecord(t1, st);
+        e = hipStreamSynchronize(st);
+        if (e != hipSuccess)
+            return hip_fail(e, fn, "Failed to synchronize after the sweeps.",
+                            NOVA_ERROR_DEVICE_SYNCHRONIZE);
+        vi->currentHorizon += sweeps;
+        return NOVA_SUCCESS;
+    }
     const unsigned long long layout = plan.chunked ? plan.chunked->serial
                                                    : (plan.sorted ? plan.sorted->serial : 0ull);
     const void *key[8] = {mdp->d_S, mdp->d_T, mdp->d_R, vi->d_V, vi->d_VPrime, vi->d_pi,

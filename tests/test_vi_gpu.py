@@ -89,6 +89,67 @@ def test_bitwise_vs_oracle(oracle, n, m, ns, horizon, seed):
     assert err < 1e-4
 
 
+# 4 (2 n + n m + n m ns) + 2 n m ns bytes of LDS hold a model for the one-launch run: at
+# m = ns = 1 the largest n is 9,102
+@pytest.mark.parametrize("n,m,ns,sweeps", [
+    (1, 1, 1, 2), (3, 64, 1, 5), (2, 100, 3, 4), (15, 65, 2, 3), (64, 16, 9, 7), (511, 2, 8, 6),
+    (1023, 3, 5, 5), (1025, 2, 7, 4), (9102, 1, 1, 3), (9103, 1, 1, 3), (900, 5, 6, 2),
+])
+def test_resident_run_vs_oracle(oracle, monkeypatch, n, m, ns, sweeps):
+    """Runs of sweeps inside one workgroup (and the first sizes past it): V and pi equal the
+    oracle's, and the previous iterate is left where the next sweep's partner buffer is."""
+    import torch
+    rng = np.random.default_rng(n + m + ns)
+    w = synth.mdp_arrays(n=n, m=m, ns=min(ns, n), seed=n, gamma=0.97)
+    S = w["S"].copy()
+    cut = rng.random(S.shape[:2]) < 0.3
+    pos = rng.integers(0, S.shape[2], size=S.shape[:2])
+    for s, a in zip(*np.nonzero(cut)):
+        S[s, a, pos[s, a]] = -1
+    R = np.round(w["R"], 1).astype(np.float32)          # tied actions
+    mdp = MDP.from_arrays(S, w["T"], R, gamma=w["gamma"], horizon=sweeps)
+    mdp.initialize_gpu()
+    v0 = rng.uniform(-5, 5, n).astype(np.float32)
+    d_v0 = torch.from_numpy(v0).cuda()
+    out = {}
+    for kernel in ("", "tiled"):
+        if kernel:
+            monkeypatch.setenv("NOVA_AMD_VI_KERNEL", kernel)
+        vi = MDPValueIterationGPU(mdp, Vinitial=v0)
+        vi.run(sweeps, d_V0=d_v0.data_ptr())
+        V, pi = vi.device_values()
+        vi.currentHorizon -= 1                           # the partner buffer
+        out[kernel] = (V, pi, vi.get_policy().V_array())
+    Vo, pio = oracle.vi_run(S, w["T"], R, w["gamma"], sweeps, V0=v0)
+    prev, _ = oracle.vi_run(S, w["T"], R, w["gamma"], sweeps - 1, V0=v0)
+    for V, pi, last in out.values():
+        assert np.array_equal(bits(V), bits(Vo)) and np.array_equal(pi, pio)
+        assert np.array_equal(bits(last), bits(prev))
+
+
+def test_resident_run_nan_and_infinities(monkeypatch):
+    """A NaN at action 0 stays, one at a later action is never taken, all -inf takes action 0:
+    the same in the one-launch run and in separate sweeps."""
+    n, m, ns = 40, 5, 2
+    w = synth.mdp_arrays(n=n, m=m, ns=ns, seed=1, gamma=0.9)
+    R = w["R"].copy()
+    R[3, 0] = np.nan
+    R[5, 2] = np.nan
+    R[7, :] = -np.inf
+    R[9, 3] = np.inf
+    mdp = MDP.from_arrays(w["S"], w["T"], R, gamma=0.9, horizon=2)
+    mdp.initialize_gpu()
+    got = []
+    for kernel in ("", "tiled"):
+        if kernel:
+            monkeypatch.setenv("NOVA_AMD_VI_KERNEL", kernel)
+        got.append(solve_gpu(mdp))
+    assert np.array_equal(np.isnan(got[0][0]), np.isnan(got[1][0]))
+    fine = ~np.isnan(got[0][0])
+    assert np.array_equal(bits(got[0][0][fine]), bits(got[1][0][fine]))
+    assert np.array_equal(got[0][1], got[1][1])
+
+
 def test_run_gpu_matches_updates(oracle):
     """mdp_vi_run_gpu (graph of sweeps, restart from a device V0) equals repeated updates."""
     import torch
