@@ -33,7 +33,9 @@ namespace nova_amd {
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kTileRows = 2048;   // (s,a) rows whose Q values a workgroup stages in LDS
+constexpr int kTileRows = 2048;   // most (s,a) rows whose Q values a workgroup stages in LDS
+constexpr unsigned kTileRowsSmall = 128, kTileRowsLarge = 512;   // rows per tile (vi_plan)
+constexpr unsigned kTileSpread = 131072;   // models below this many rows take the small tiles
 constexpr int kUnroll = 8;        // rows in flight per lane group (8 measured ~4% faster than 4)
 
 typedef int int4v __attribute__((ext_vector_type(4)));
@@ -1353,7 +1355,14 @@ static ViPlan vi_plan(const nova::MDP *mdp, const nova::MDPVIGPU *vi)
             p.tiled = tiled_for<1>(pow2_at_least(ns));
     }
     if (p.tiled) {
-        p.statesPerTile = kTileRows / m;
+        // Small tiles spread a small model over the CUs (at 2,048 rows a 900-state model has three
+        // workgroups); from about two workgroups of 512 rows per CU on, larger tiles keep more
+        // rows of a lane group in flight. us per sweep at 2,048 / 512 / 128 rows:
+        // n = 900, m = 5, ns = 5: 32.5 / 9.8 / 5.4; n = 10,000, m = 7, ns = 9: 103 / 27.5 / 9.2;
+        // n = 30,000, m = 8, ns = 16: 32.6 / 16.6 / 21.2; n = 200,000, m = 6, ns = 7: 58 / 58 / 58
+        const size_t rows = (size_t)n * m;
+        const unsigned tileRows = rows < (size_t)kTileSpread ? kTileRowsSmall : kTileRowsLarge;
+        p.statesPerTile = std::max(1u, tileRows / m);
         p.grid = (n + p.statesPerTile - 1) / p.statesPerTile;
     } else {
         p.grid = (n + kBlock - 1) / kBlock;
