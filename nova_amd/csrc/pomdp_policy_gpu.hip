@@ -26,6 +26,7 @@
 //    b' and reports NOVA_WARNING_INVALID_BELIEF, as the reference returns it.
 #include <algorithm>
 #include <climits>
+#include <cstdint>
 #include <cstring>
 #include <mutex>
 #include <vector>
@@ -154,6 +155,227 @@ __global__ __launch_bounds__(256) void alpha_value_merge(unsigned k, unsigned ti
     act[i] = none ? 0u : pi[bj];
     if (jOut)
         jOut[i] = none ? -1 : bj;
+}
+
+// The same for few beliefs: one wave per tile of 16 alphas x 4 X beliefs, each lane one alpha and
+// X beliefs, so that a call of a few beliefs spreads over many CUs where alpha_value_exact has
+// one workgroup per 64 alphas. A lane's sums are serial chains over the states (the reference's
+// order), so what bounds a call is that chain and the loads that feed it: the wave requests the
+// next CH states of its rows into registers before it sums the current CH from LDS (rows padded
+// by 4 floats: the 16 alphas' 16-byte reads fall on distinct banks, the beliefs' are
+// broadcasts). One wave per workgroup: its LDS needs no barrier, only the order of its own
+// accesses. VEC: rows 16-byte aligned (n % 4 == 0).
+constexpr unsigned kFewAlphas = 16;
+
+template <int X, int CH, bool VEC>
+__global__ __launch_bounds__(64) void alpha_value_few(unsigned k, unsigned n, unsigned r,
+        const float *__restrict__ B, const float *__restrict__ G, float *__restrict__ partV,
+        int *__restrict__ partJ)
+{
+    constexpr int kRows = (int)kFewAlphas + 4 * X, kStride = CH + 4;
+    // a lane's loads per chunk: VEC takes float4s numbered row-major over the tile, else words
+    constexpr int kAcross = VEC ? CH / 4 : CH;
+    constexpr int kPer = kAcross * kRows / 64;
+    __shared__ __attribute__((aligned(16))) float buf[kRows * kStride];
+    const unsigned lane = threadIdx.x, al = lane % kFewAlphas, bl = lane / kFewAlphas;
+    const unsigned j0 = blockIdx.y * kFewAlphas, i0 = blockIdx.x * 4 * X;
+    // row q of the tile: alphas, then beliefs; rows past r or k repeat the last one
+    auto rowOf = [&](unsigned q) {
+        return q < kFewAlphas ? G + (size_t)min(j0 + q, r - 1) * n
+                              : B + (size_t)min(i0 + (q - kFewAlphas), k - 1) * n;
+    };
+    float4 pre4[VEC ? kPer : 1];
+    float pre[VEC ? 1 : kPer];
+    // states past n are zeros in both operands: their products add +0
+    auto load = [&](unsigned s0) {
+#pragma unroll
+        for (int u = 0; u < kPer; u++) {
+            const unsigned e = u * 64 + lane;
+            const float *row = rowOf(e / kAcross);
+            if constexpr (VEC) {
+                const unsigned s = s0 + e % kAcross * 4;
+                pre4[u] = s < n ? *reinterpret_cast<const float4 *>(row + s)
+                                : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            } else {
+                const unsigned s = s0 + e % kAcross;
+                pre[u] = s < n ? row[s] : 0.0f;
+            }
+        }
+    };
+    float acc[X];
+#pragma unroll
+    for (int x = 0; x < X; x++)
+        acc[x] = 0.0f;
+    load(0);
+    for (unsigned s0 = 0; s0 < n; s0 += CH) {
+#pragma unroll
+        for (int u = 0; u < kPer; u++) {
+            const unsigned e = u * 64 + lane;
+            if constexpr (VEC)
+                *reinterpret_cast<float4 *>(&buf[e / kAcross * kStride + e % kAcross * 4]) =
+                    pre4[u];
+            else
+                buf[e / kAcross * kStride + e % kAcross] = pre[u];
+        }
+        __syncthreads();
+        if (s0 + CH < n)
+            load(s0 + CH);
+        // blocks of 16 states; one belief per lane reads the next block from LDS before it sums
+        // the current one (n = 5,000: 67 -> 62 us; two beliefs per lane lose more to the
+        // registers this takes, 129 -> 141 us at n = 5,000, r = 1,024, k = 256)
+        const unsigned cnt = min((unsigned)CH, (n - s0 + 15) / 16 * 16);
+        float4 g[4], bb[X][4];
+        auto read = [&](unsigned s, float4 (&gq)[4], float4 (&bq)[X][4]) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                gq[v] = *reinterpret_cast<const float4 *>(&buf[al * kStride + s + 4 * v]);
+#pragma unroll
+                for (int x = 0; x < X; x++)
+                    bq[x][v] = *reinterpret_cast<const float4 *>(
+                        &buf[(kFewAlphas + bl * X + x) * kStride + s + 4 * v]);
+            }
+        };
+        auto sum = [&](const float4 (&gq)[4], const float4 (&bq)[X][4]) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const float g4[4] = {gq[v].x, gq[v].y, gq[v].z, gq[v].w};
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+#pragma unroll
+                    for (int x = 0; x < X; x++) {
+                        const float b4[4] = {bq[x][v].x, bq[x][v].y, bq[x][v].z, bq[x][v].w};
+                        acc[x] = __fadd_rn(acc[x], __fmul_rn(g4[e], b4[e]));
+                    }
+            }
+        };
+        if constexpr (X == 1) {
+            read(0, g, bb);
+            for (unsigned s = 0; s < cnt; s += 32) {
+                float4 g2[4], bb2[X][4];
+                read(min(s + 16, (unsigned)CH - 16), g2, bb2);
+                __builtin_amdgcn_sched_barrier(0);
+                sum(g, bb);
+                if (s + 16 < cnt) {
+                    read(min(s + 32, (unsigned)CH - 16), g, bb);
+                    __builtin_amdgcn_sched_barrier(0);
+                    sum(g2, bb2);
+                }
+            }
+        } else {
+            for (unsigned s = 0; s < cnt; s += 16) {
+                read(s, g, bb);
+                sum(g, bb);
+            }
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int x = 0; x < X; x++) {
+        const bool use = j0 + al < r && acc[x] > kLow;
+        float bv = use ? acc[x] : kLow;
+        int bj = use ? (int)(j0 + al) : INT_MAX;
+        for (int off = 8; off >= 1; off >>= 1) {
+            const float ov = __shfl_xor(bv, off, 16);
+            const int oj = __shfl_xor(bj, off, 16);
+            if (better(ov, oj, bv, bj)) {
+                bv = ov;
+                bj = oj;
+            }
+        }
+        const unsigned i = i0 + bl * X + x;
+        if (al == 0 && i < k) {
+            partV[(size_t)blockIdx.y * k + i] = bv;
+            partJ[(size_t)blockIdx.y * k + i] = bj;
+        }
+    }
+}
+
+// alpha_value_merge with one wave per belief, for few beliefs and many tiles.
+__global__ __launch_bounds__(64) void alpha_value_merge_few(unsigned k, unsigned tiles,
+        const float *__restrict__ partV, const int *__restrict__ partJ,
+        const unsigned *__restrict__ pi, float *__restrict__ V, unsigned *__restrict__ act,
+        int *__restrict__ jOut)
+{
+    const unsigned i = blockIdx.x;
+    float bv = kLow;
+    int bj = INT_MAX;
+    for (unsigned tl = threadIdx.x; tl < tiles; tl += 64) {
+        const float v = partV[(size_t)tl * k + i];
+        const int j = partJ[(size_t)tl * k + i];
+        if (better(v, j, bv, bj)) {
+            bv = v;
+            bj = j;
+        }
+    }
+    for (int off = 32; off >= 1; off >>= 1) {
+        const float ov = __shfl_xor(bv, off);
+        const int oj = __shfl_xor(bj, off);
+        if (better(ov, oj, bv, bj)) {
+            bv = ov;
+            bj = oj;
+        }
+    }
+    if (threadIdx.x != 0)
+        return;
+    const bool none = (bj == INT_MAX) || !(bv > kLow);
+    V[i] = none ? kLow : bv;
+    act[i] = none ? 0u : pi[bj];
+    if (jOut)
+        jOut[i] = none ? -1 : bj;
+}
+
+template <int X, int CH>
+void launch_few(unsigned k, unsigned n, unsigned r, const float *B, const float *G, float *partV,
+                int *partJ, hipStream_t st)
+{
+    const bool vec = n % 4 == 0 && ((reinterpret_cast<uintptr_t>(B) |
+                                     reinterpret_cast<uintptr_t>(G)) & 15u) == 0;
+    const dim3 g((k + 4 * X - 1) / (4 * X), (r + kFewAlphas - 1) / kFewAlphas);
+    if (vec)
+        hipLaunchKernelGGL((alpha_value_few<X, CH, true>), g, dim3(64), 0, st, k, n, r, B, G,
+                           partV, partJ);
+    else
+        hipLaunchKernelGGL((alpha_value_few<X, CH, false>), g, dim3(64), 0, st, k, n, r, B, G,
+                           partV, partJ);
+}
+
+// Beliefs per lane of alpha_value_few for a call, or 0 where alpha_value_exact is the faster:
+// one while that gives at most 2,048 waves (two per SIMD), then two, until alpha_value_exact has
+// a workgroup per CU and more. us of a call, 0 / 1 / 2 beliefs per lane: n = 5,000, r = 1,024:
+// k = 4: 602 / 62 / 90; k = 256: 630 / 208 / 131; k = 2,048: 595 / 1,189 / 745. n = 20,000,
+// r = 4,096: k = 1: 2,400 / 204 / 311; k = 64: 2,480 / 829 / 460; k = 256: 2,470 / 2,490 /
+// 1,540; k = 512: 2,290 / 4,660 / 3,150.
+constexpr size_t kFewPairs = 5u << 18;       // most (belief, alpha) pairs, 1.25 Mi
+
+unsigned few_beliefs(unsigned k, unsigned r)
+{
+    if ((size_t)k * r > kFewPairs || r > 65535u * kFewAlphas)   // (the grid's y extent)
+        return 0;
+    const size_t waves = (size_t)((k + 3) / 4) * ((r + kFewAlphas - 1) / kFewAlphas);
+    return waves <= 2048 ? 1 : 2;
+}
+
+// Alphas per partial of the exact mode.
+inline unsigned exact_tile(unsigned few) { return few ? kFewAlphas : (unsigned)kVT; }
+
+void launch_exact(unsigned few, unsigned k, unsigned n, unsigned r, const float *B,
+                  const float *G, const unsigned *pi, float *partV, int *partJ, float *V,
+                  unsigned *act, int *jOut, hipStream_t st)
+{
+    const unsigned tiles = (r + exact_tile(few) - 1) / exact_tile(few);
+    if (few == 0) {
+        hipLaunchKernelGGL(alpha_value_exact, dim3((k + kVT - 1) / kVT, tiles), dim3(kVThreads),
+                           0, st, k, n, r, B, G, partV, partJ);
+        hipLaunchKernelGGL(alpha_value_merge, dim3((k + 255) / 256), dim3(256), 0, st, k, tiles,
+                           partV, partJ, pi, V, act, jOut);
+        return;
+    }
+    if (few == 1)
+        launch_few<1, 256>(k, n, r, B, G, partV, partJ, st);
+    else
+        launch_few<2, 128>(k, n, r, B, G, partV, partJ, st);
+    hipLaunchKernelGGL(alpha_value_merge_few, dim3(k), dim3(64), 0, st, k, tiles, partV, partJ,
+                       pi, V, act, jOut);
 }
 
 __global__ __launch_bounds__(256) void fill_ones(unsigned count, float *__restrict__ x)
@@ -604,7 +826,8 @@ extern "C" int nova_amd_alpha_vectors_value_and_action_gpu(unsigned int n, unsig
     std::lock_guard<std::mutex> lock(g_valueMutex);
     hipStream_t st = stream();
     const bool exact = precision == 0;
-    const unsigned tileW = exact ? (unsigned)kVT : (unsigned)kGT;
+    const unsigned few = exact ? few_beliefs(k, r) : 0;
+    const unsigned tileW = exact ? exact_tile(few) : (unsigned)kGT;
     const unsigned colTiles = (r + tileW - 1) / tileW;
     const unsigned rowTiles = (k + kGT - 1) / kGT;
     const size_t inSize = precision == 2 ? sizeof(__bf16) : sizeof(float);
@@ -628,8 +851,7 @@ extern "C" int nova_amd_alpha_vectors_value_and_action_gpu(unsigned int n, unsig
     hipError_t e = hipSuccess;
     if (exact) {
         g_valueShape = DenseShape();   // the partials may overwrite the dense operands' padding
-        hipLaunchKernelGGL(alpha_value_exact, dim3((k + kVT - 1) / kVT, colTiles),
-                           dim3(kVThreads), 0, st, k, n, r, d_B, d_Gamma, partV, partJ);
+        launch_exact(few, k, n, r, d_B, d_Gamma, d_pi, partV, partJ, d_V, d_action, d_alpha, st);
     } else {
         void *A = c + 2 * bPart, *Gi = c + 2 * bPart + bA;
         float *ones = reinterpret_cast<float *>(c + 2 * bPart + bA + bG);
@@ -694,8 +916,9 @@ extern "C" int nova_amd_alpha_vectors_value_and_action_gpu(unsigned int n, unsig
                                static_cast<const float *>(Gi), ones, partV, partJ);
         }
     }
-    hipLaunchKernelGGL(alpha_value_merge, dim3((k + 255) / 256), dim3(256), 0, st, k, colTiles,
-                       partV, partJ, d_pi, d_V, d_action, d_alpha);
+    if (!exact)
+        hipLaunchKernelGGL(alpha_value_merge, dim3((k + 255) / 256), dim3(256), 0, st, k,
+                           colTiles, partV, partJ, d_pi, d_V, d_action, d_alpha);
     if (e == hipSuccess)
         e = hipGetLastError();
     if (e == hipSuccess)
@@ -778,8 +1001,8 @@ extern "C" int nova_amd_alpha_vectors_value_and_action_noalloc_gpu(unsigned int 
         NOVA_ERR(fn, "Invalid arguments (n, r, k > 0, r <= 4,194,240; device arrays).");
         return NOVA_ERROR_INVALID_DATA;
     }
-    const size_t colTiles = (r + kVT - 1) / kVT;
-    const size_t bPart = up256(colTiles * k * sizeof(float));
+    size_t colTiles = (r + kVT - 1) / kVT;
+    size_t bPart = up256(colTiles * k * sizeof(float));
     if (2 * bPart > kNoAllocScratchBytes) {
         NOVA_ERR(fn, "ceil(r / 64) * k exceeds the 16 MiB scratch array (at most 2,097,152 "
                      "(belief, 64-alpha tile) partials per call).");
@@ -788,13 +1011,19 @@ extern "C" int nova_amd_alpha_vectors_value_and_action_noalloc_gpu(unsigned int 
     char *c = static_cast<char *>(scratch_address(fn));
     if (c == nullptr)
         return NOVA_ERROR_KERNEL_EXECUTION;
+    // the narrower tiles of few beliefs have four times the partials: only where they fit too
+    unsigned few = few_beliefs(k, r);
+    if (few) {
+        colTiles = (r + kFewAlphas - 1) / kFewAlphas;
+        if (2 * up256(colTiles * k * sizeof(float)) <= kNoAllocScratchBytes)
+            bPart = up256(colTiles * k * sizeof(float));
+        else
+            few = 0;
+    }
     hipStream_t st = stream();
     float *partV = reinterpret_cast<float *>(c);
     int *partJ = reinterpret_cast<int *>(c + bPart);
-    hipLaunchKernelGGL(alpha_value_exact, dim3((k + kVT - 1) / kVT, (unsigned)colTiles),
-                       dim3(kVThreads), 0, st, k, n, r, d_B, d_Gamma, partV, partJ);
-    hipLaunchKernelGGL(alpha_value_merge, dim3((k + 255) / 256), dim3(256), 0, st, k,
-                       (unsigned)colTiles, partV, partJ, d_pi, d_V, d_action, d_alpha);
+    launch_exact(few, k, n, r, d_B, d_Gamma, d_pi, partV, partJ, d_V, d_action, d_alpha, st);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess)
         e = hipStreamSynchronize(st);

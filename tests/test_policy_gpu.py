@@ -60,6 +60,43 @@ def test_exact_bitwise_vs_oracle(oracle, k, n, r):
     print("exact value/action: k=%d n=%d r=%d bit-identical" % (k, n, r), flush=True)
 
 
+@pytest.mark.parametrize("k,n,r,offset", [
+    (1, 1, 1, 0), (4, 16, 16, 0), (5, 17, 17, 0), (3, 255, 15, 0), (9, 256, 33, 0),
+    (2, 260, 64, 1), (7, 513, 100, 0), (1030, 36, 130, 0), (2049, 130, 66, 3), (600, 20, 2200, 0),
+])
+def test_exact_few_beliefs_bitwise(oracle, k, n, r, offset):
+    """The one-wave tiles of calls with few (belief, alpha) pairs: one and two beliefs per lane,
+    rows aligned to 16 bytes or not (n odd, or arrays offset by some floats), partial tiles."""
+    import torch
+    from nova_amd import _abi
+    G, pi, B = instance(k, n, r, seed=7 * k + n + r)
+    if r > 3:
+        G[r - 1] = G[1]
+    if n > 2:
+        G[0, 1] = np.inf          # (an infinity times a zero belief entry is a NaN, never chosen)
+    Gt = torch.zeros(r * n + offset, device="cuda")
+    Bt = torch.zeros(k * n + offset, device="cuda")
+    Gt[offset:] = torch.from_numpy(G).reshape(-1)
+    Bt[offset:] = torch.from_numpy(B).reshape(-1)
+    pt = torch.from_numpy(pi.astype(np.int32)).cuda()
+    V = torch.empty(k, device="cuda")
+    a = torch.empty(k, dtype=torch.int32, device="cuda")
+    j = torch.empty(k, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    lib = _abi.load()
+    for entry, extra in ((lib.nova_amd_alpha_vectors_value_and_action_gpu, [0]),
+                         (lib.nova_amd_alpha_vectors_value_and_action_noalloc_gpu, [])):
+        V.zero_()
+        torch.cuda.synchronize()
+        assert entry(n, r, Gt.data_ptr() + 4 * offset, pt.data_ptr(), k,
+                     Bt.data_ptr() + 4 * offset, *extra, V.data_ptr(), a.data_ptr(),
+                     j.data_ptr()) == 0
+        Vh, ah, jh = V.cpu().numpy(), a.cpu().numpy(), j.cpu().numpy()
+        for i in range(0, k, max(1, k // 60)):
+            vo, ao, jo = oracle.alpha_value(G, pi, B[i])
+            assert bits(np.float32(vo)) == bits(Vh[i]) and ao == ah[i] and jo == jh[i], i
+
+
 def test_exact_no_alpha_above_sentinel():
     """Every value at or below -1e10: V = -1e10, action 0 and alpha -1 (the reference leaves
     Vb and a at their initial values). Exact and fp32 only: in bf16 the sentinel itself rounds
