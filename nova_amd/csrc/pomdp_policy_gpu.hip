@@ -385,7 +385,8 @@ __global__ __launch_bounds__(256) void fill_ones(unsigned count, float *__restri
         x[i] = 1.0f;
 }
 
-// Belief updates in three kernels, each sum in the reference's order:
+// Belief updates in three kernels (four for many triples: belief_tiles, belief_update_tiles in
+// the place of the first), each sum in the reference's order:
 //   belief_update_batch: one workgroup per triple q; b is staged in LDS. Wave w takes blocks
 //     of 64 consecutive states s'. The block's predecessor entries (contiguous in the lists)
 //     are read 64 at a time, coalesced, and their products T * b(s) formed into the wave's LDS
@@ -475,13 +476,18 @@ __global__ __launch_bounds__(kUB) void belief_update_batch(unsigned n, unsigned 
 
 // The k triples grouped by action (a counting sort in one workgroup; invalid actions last).
 // The order within an action is whatever the atomics give: each triple's result does not
-// depend on when it runs.
+// depend on when it runs. tiles (nullable) receives the groups cut into tiles of at most
+// kTileT triples of one action, (action, first position in order, triples, 0); the entries
+// past the last tile, up to maxTiles, get 0 triples.
 constexpr unsigned kOrderMaxM = 4096;
+constexpr size_t kOrderListBytes = (size_t)4 << 20;
+constexpr unsigned kTileT = 32;
 
 __global__ __launch_bounds__(1024) void order_by_action(unsigned k, unsigned m,
-        const unsigned *__restrict__ act, unsigned *__restrict__ order)
+        const unsigned *__restrict__ act, unsigned *__restrict__ order, uint4 *__restrict__ tiles,
+        unsigned maxTiles)
 {
-    __shared__ unsigned cnt[kOrderMaxM + 1];
+    __shared__ unsigned cnt[kOrderMaxM + 1], first[kOrderMaxM + 1];
     const unsigned t = threadIdx.x;
     for (unsigned x = t; x <= m; x += 1024)
         cnt[x] = 0;
@@ -490,59 +496,239 @@ __global__ __launch_bounds__(1024) void order_by_action(unsigned k, unsigned m,
         atomicAdd(&cnt[min(act[q], m)], 1u);
     __syncthreads();
     if (t == 0) {
-        unsigned run = 0;
+        unsigned run = 0, tile = 0;
         for (unsigned x = 0; x <= m; x++) {
             const unsigned c = cnt[x];
             cnt[x] = run;
+            first[x] = tile;
             run += c;
+            tile += (c + kTileT - 1) / kTileT;
         }
+    }
+    __syncthreads();
+    if (tiles) {
+        const unsigned used = first[m];
+        for (unsigned x = t; x < m; x += 1024)
+            for (unsigned q = cnt[x], i = first[x]; q < cnt[x + 1]; q += kTileT, i++)
+                tiles[i] = make_uint4(x, q, min(kTileT, cnt[x + 1] - q), 0u);
+        for (unsigned i = used + t; i < maxTiles; i += 1024)
+            tiles[i] = make_uint4(0u, 0u, 0u, 0u);
     }
     __syncthreads();
     for (unsigned q = t; q < k; q += 1024)
         order[atomicAdd(&cnt[min(act[q], m)], 1u)] = q;
 }
 
+// Many updates: the beliefs of a tile of kTileT triples of one action are laid out state-major,
+// BT[tile][s][triple], so that one predecessor entry (s, T) serves all of them with one
+// 128-byte row. belief_update_batch re-reads the action's whole list (6 or 8 bytes an entry)
+// for every belief; here a list is read once per tile and a belief costs 4 coalesced bytes an
+// entry, from the L2 that holds its tile (n x 128 bytes). Sums run over the same lists in the
+// same order, products and sums rounded as there.
+constexpr unsigned kTileS = 128;         // states per workgroup of the two kernels
+constexpr unsigned kTileThreads = 256;
+
+__global__ __launch_bounds__(kTileThreads) void belief_tiles(unsigned n,
+        const uint4 *__restrict__ tiles, const unsigned *__restrict__ order,
+        const unsigned *__restrict__ rowOf, const float *__restrict__ B, float *__restrict__ BT)
+{
+    __shared__ float buf[kTileT][kTileS + 1];
+    const uint4 tile = tiles[blockIdx.y];
+    if (tile.z == 0)
+        return;
+    const unsigned t = threadIdx.x, s0 = blockIdx.x * kTileS;
+    constexpr unsigned kPer = kTileT * kTileS / kTileThreads;
+    float v[kPer];
+#pragma unroll
+    for (unsigned u = 0; u < kPer; u++) {
+        const unsigned x = u * kTileThreads + t, i = x / kTileS, s = s0 + x % kTileS;
+        v[u] = 0.0f;
+        if (i < tile.z && s < n) {
+            const unsigned q = order[tile.y + i];
+            v[u] = B[(size_t)(rowOf ? rowOf[q] : q) * n + s];
+        }
+    }
+#pragma unroll
+    for (unsigned u = 0; u < kPer; u++) {
+        const unsigned x = u * kTileThreads + t;
+        buf[x / kTileS][x % kTileS] = v[u];
+    }
+    __syncthreads();
+    float *out = BT + ((size_t)blockIdx.y * n + s0) * kTileT;
+#pragma unroll
+    for (unsigned u = 0; u < kPer; u++) {
+        const unsigned x = u * kTileThreads + t, s = x / kTileT, i = x % kTileT;
+        if (s0 + s < n)
+            out[x] = buf[i][s];
+    }
+}
+
+// The unnormalised updates of the tiles: 8 lanes per state s', each holding four triples; a
+// lane walks the state's predecessors kTileE at a time (the next ones' indices and factors
+// requested before this round's beliefs are summed), multiplies by O[a, s', o] and leaves the
+// products in LDS, from where the triples' rows are written past the caches. At n = 20,000,
+// ns = 8 a chunk of 48 tiles takes 133 us (7.4 TB/s of gathered rows, of which about 4.7 TB/s
+// pass L2: the beliefs, O and the rows written, each as large); 16 triples a tile take 196 us per
+// 48, staging the lists in LDS 160 us (fewer workgroups fit), 8 entries at a time 151 us. Workgroups are dealt to the XCDs
+// in turn: workgroup b takes a tile of XCD b mod 8, so that the workgroups running together on
+// an XCD share one tile's BT.
+constexpr unsigned kTileE = 4;
+constexpr size_t kTileBytes = (size_t)128 << 20;     // state-major beliefs of a chunk of tiles
+
+template <typename IDX>
+__global__ __launch_bounds__(kTileThreads) void belief_update_tiles(unsigned n, unsigned z,
+        unsigned blocks, const uint4 *__restrict__ tiles, const unsigned *__restrict__ order,
+        const unsigned *__restrict__ pstart, const IDX *__restrict__ pS,
+        const float *__restrict__ pT, const float *__restrict__ O,
+        const unsigned *__restrict__ obs, const float *__restrict__ BT, float *__restrict__ Bp)
+{
+    __shared__ float buf[kTileT][kTileS + 1];
+    __shared__ unsigned row[kTileT];         // the triple's row of Bp, or ~0 when it has none
+    const unsigned b = blockIdx.x / 8, slot = b / blocks * 8 + blockIdx.x % 8;
+    const uint4 tile = tiles[slot];
+    if (tile.z == 0)
+        return;
+    const unsigned t = threadIdx.x, s0 = b % blocks * kTileS, a = tile.x;
+    constexpr unsigned kL = kTileT / 4;      // lanes per state
+    const unsigned l = t % kL, first = 4 * l;
+    unsigned o[4];
+#pragma unroll
+    for (unsigned e = 0; e < 4; e++) {
+        // (an observation out of range: no row is written, belief_norms reports it)
+        const unsigned ob = first + e < tile.z ? obs[order[tile.y + first + e]] : z;
+        o[e] = min(ob, z - 1);
+        if (t < kL)
+            row[first + e] = ob < z ? order[tile.y + first + e] : ~0u;
+    }
+    const unsigned *ps = pstart + (size_t)a * (n + 1);
+    const float *Oa = O + (size_t)a * n * z;
+    const float4 *bt = reinterpret_cast<const float4 *>(BT + (size_t)slot * n * kTileT) + l;
+    for (unsigned s = t / kL; s < kTileS; s += kTileThreads / kL) {
+        const unsigned sp = s0 + s;
+        if (sp >= n)
+            break;
+        const unsigned lo = ps[sp], hi = ps[sp + 1];
+        float u[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (lo < hi) {
+            IDX si[kTileE];
+            float tv[kTileE];
+            auto request = [&](unsigned x) {
+#pragma unroll
+                for (unsigned e = 0; e < kTileE; e++) {
+                    const unsigned at = min(x + e, hi - 1);
+                    si[e] = pS[at];
+                    tv[e] = pT[at];
+                }
+            };
+            request(lo);
+            for (unsigned x = lo; x < hi; x += kTileE) {
+                float4 bv[kTileE];
+                float tc[kTileE];
+#pragma unroll
+                for (unsigned e = 0; e < kTileE; e++) {
+                    bv[e] = bt[(size_t)si[e] * (kTileT / 4)];
+                    tc[e] = tv[e];
+                }
+                if (x + kTileE < hi)
+                    request(x + kTileE);
+#pragma unroll
+                for (unsigned e = 0; e < kTileE; e++)
+                    if (x + e < hi) {
+                        u[0] = __fadd_rn(u[0], __fmul_rn(tc[e], bv[e].x));
+                        u[1] = __fadd_rn(u[1], __fmul_rn(tc[e], bv[e].y));
+                        u[2] = __fadd_rn(u[2], __fmul_rn(tc[e], bv[e].z));
+                        u[3] = __fadd_rn(u[3], __fmul_rn(tc[e], bv[e].w));
+                    }
+            }
+        }
+#pragma unroll
+        for (unsigned e = 0; e < 4; e++)
+            buf[first + e][s] = __fmul_rn(u[e], Oa[(size_t)sp * z + o[e]]);
+    }
+    __syncthreads();
+    constexpr unsigned kPer = kTileT * kTileS / kTileThreads;
+#pragma unroll
+    for (unsigned v = 0; v < kPer; v++) {
+        const unsigned x = v * kTileThreads + t, i = x / kTileS, s = x % kTileS;
+        if (s0 + s < n && row[i] != ~0u)
+            __builtin_nontemporal_store(buf[i][s], Bp + (size_t)row[i] * n + s0 + s);
+    }
+}
+
 constexpr unsigned kNormT = 16;          // triples per workgroup of belief_norms
 constexpr unsigned kNormC = 512;         // states per chunk
 constexpr unsigned kNormLoaders = 256;   // lanes of waves 1-4, 32 values each per chunk
 
+// The normaliser is one serial sum per triple: waves 1-4 stream chunks of the 16 rows into one
+// buffer (coalesced, all 32 loads of a lane in flight together) while lanes 0-15 of wave 0 add
+// the other buffer's chunk into their triple's sum, in order. What bounds it is that chain of
+// adds: 16 values are read from LDS as four 16-byte words while the 16 before are added (one
+// word at a time, each add waited for its own LDS read: 593 us for 16,384 triples of 20,000
+// states, now 519 us, at 2.5 TB/s). Rows are padded to 516 floats so that the 16 lanes' reads fall on distinct
+// banks; values past n are zeros, which leave the sum (never -0) as it is.
 __global__ __launch_bounds__(64 + kNormLoaders) void belief_norms(unsigned n, unsigned m,
         unsigned z, unsigned k, const unsigned *__restrict__ act,
         const unsigned *__restrict__ obs, const float *__restrict__ Bp,
         float *__restrict__ norms, int *__restrict__ status)
 {
-    // waves 1-4 stream chunks of the 16 rows into one buffer (coalesced, all 32 loads of a
-    // lane in flight together) while lanes 0-15 of wave 0 add the other buffer's chunk into
-    // their triple's sum, in order; rows padded to 513 floats so that the 16 summing lanes
-    // read distinct banks
     constexpr unsigned kPer = kNormT * kNormC / kNormLoaders;
-    __shared__ float buf[2][kNormT][kNormC + 1];
+    __shared__ __attribute__((aligned(16))) float buf[2][kNormT][kNormC + 4];
     const unsigned t = threadIdx.x, q0 = blockIdx.x * kNormT;
-    auto load = [&](unsigned c0, unsigned which) {
-        float v[kPer];
+    // the loaders' values: requested one chunk before they are written to LDS, two before they
+    // are summed
+    float v[kPer];
+    auto request = [&](unsigned c0) {
 #pragma unroll
         for (unsigned u = 0; u < kPer; u++) {
             const unsigned e = (t - 64) + kNormLoaders * u, j = e / kNormC, i = e % kNormC;
             v[u] = (q0 + j < k && c0 + i < n) ? Bp[(size_t)(q0 + j) * n + c0 + i] : 0.0f;
         }
+    };
+    auto place = [&](unsigned which) {
 #pragma unroll
         for (unsigned u = 0; u < kPer; u++) {
             const unsigned e = (t - 64) + kNormLoaders * u;
             buf[which][e / kNormC][e % kNormC] = v[u];
         }
     };
-    if (t >= 64)
-        load(0, 0);
+    if (t >= 64) {
+        request(0);
+        place(0);
+        request(kNormC);
+    }
     __syncthreads();
     float c = 0.0f;
     unsigned cur = 0;
     for (unsigned c0 = 0; c0 < n; c0 += kNormC, cur ^= 1) {
-        if (t >= 64 && c0 + kNormC < n)
-            load(c0 + kNormC, cur ^ 1);
+        if (t >= 64 && c0 + kNormC < n) {
+            place(cur ^ 1);
+            request(c0 + 2 * kNormC);        // (zeros past n)
+        }
         if (t < kNormT) {
-            const unsigned cnt = min(kNormC, n - c0);
-            for (unsigned i = 0; i < cnt; i++)
-                c = __fadd_rn(c, buf[cur][t][i]);
+            const float4 *row = reinterpret_cast<const float4 *>(buf[cur][t]);
+            const unsigned end = (min(kNormC, n - c0) + 15) / 16 * 4;
+            float4 x[4];
+#pragma unroll
+            for (unsigned e = 0; e < 4; e++)
+                x[e] = row[e];
+            for (unsigned i = 0; i < end; i += 4) {
+                float4 w[4];
+                const unsigned next = min(i + 4, kNormC / 4 - 4);
+#pragma unroll
+                for (unsigned e = 0; e < 4; e++)
+                    w[e] = row[next + e];
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (unsigned e = 0; e < 4; e++) {
+                    c = __fadd_rn(c, x[e].x);
+                    c = __fadd_rn(c, x[e].y);
+                    c = __fadd_rn(c, x[e].z);
+                    c = __fadd_rn(c, x[e].w);
+                }
+#pragma unroll
+                for (unsigned e = 0; e < 4; e++)
+                    x[e] = w[e];
+            }
         }
         __syncthreads();
     }
@@ -749,6 +935,20 @@ static int pred_lists(const nova::POMDP *p, const char *fn)
 
 namespace nova_amd {
 
+// Whether a batch of updates goes through the tiles of kTileT triples: where one workgroup per
+// triple is too slow a walk (n from 8,192 on) or the batch is large, and the actions' groups
+// fill their tiles well enough (a tile costs about the same with 1 triple as with 32). us of a
+// call, workgroup per triple / tiles: n = 20,000, m = 16: k = 128: 796 / 783, k = 1,024:
+// 1,007 / 896, k = 16,384: 6,260 / 3,730; n = 10,000, m = 8: k = 1,024: 306 / 251; n = 3,001,
+// m = 7: k = 512: 88 / 99, k = 4,096: 171 / 151; n = 500, m = 4: k = 16,384: 166 / 124.
+static bool update_tiled(unsigned k, unsigned n, unsigned m, unsigned z)
+{
+    if (m > kOrderMaxM || (size_t)n * kTileT * 4 >= ((size_t)1 << 32) ||
+            (size_t)n * z >= ((size_t)1 << 30))      // (32-bit byte offsets)
+        return false;
+    return (n >= 8192 && (k >= 8 * m || m <= 16)) || (k >= 4096 && k >= 32 * m);
+}
+
 // tau(b, a, o) for k triples whose beliefs are rows rowOf[q] of B (rowOf null: row q), bit for
 // bit nova's pomdp_belief_update_cpu; shared by the batched entry point and the GPU PEMA.
 int belief_update_rows(const nova::POMDP *pomdp, unsigned k, const float *d_B,
@@ -766,32 +966,63 @@ int belief_update_rows(const nova::POMDP *pomdp, unsigned k, const float *d_B,
     int rc = pred_lists(pomdp, fn);
     if (rc != NOVA_SUCCESS)
         return rc;
+    const unsigned n = pomdp->n, m = pomdp->m;
+    // tiles of one action's triples: at most ceil(k / kTileT) + m of them, in chunks whose
+    // state-major beliefs take kTileBytes (and at least a tile per XCD)
+    const bool tiled = update_tiled(k, n, m, pomdp->z);
+    const unsigned blocks = (n + kTileS - 1) / kTileS;
+    const size_t tileBytes = sizeof(float) * kTileT * (size_t)n;
+    const unsigned maxTiles = tiled ? ((k + kTileT - 1) / kTileT + m + 7) / 8 * 8 : 0;
+    const unsigned chunkTiles =
+        (unsigned)std::min<size_t>(maxTiles, std::max<size_t>(kTileBytes / tileBytes / 8, 1) * 8);
+    const size_t normBytes = up256(sizeof(float) * (size_t)k);
+    const size_t orderBytes = up256(sizeof(unsigned) * (size_t)k);
+    const size_t listBytes = up256(sizeof(uint4) * (size_t)maxTiles);
     void *mem = nullptr;
-    const size_t normBytes = (sizeof(float) * (size_t)k + 255) / 256 * 256;
-    rc = arena_get(g_updateArena, normBytes + sizeof(unsigned) * (size_t)k, fn, mem);
+    rc = arena_get(g_updateArena, normBytes + orderBytes + listBytes + tileBytes * chunkTiles, fn,
+                   mem);
     if (rc != NOVA_SUCCESS)
         return rc;
-    float *norms = static_cast<float *>(mem);
-    unsigned *order = pomdp->m <= kOrderMaxM
-                      ? reinterpret_cast<unsigned *>(static_cast<char *>(mem) + normBytes)
-                      : nullptr;
+    char *c = static_cast<char *>(mem);
+    float *norms = reinterpret_cast<float *>(c);
+    // without tiles, grouping by action pays only where the predecessor lists exceed an L2
+    const bool grouped = tiled || (m <= kOrderMaxM &&
+                                   (size_t)n * m * pomdp->ns * sizeof(float) > kOrderListBytes);
+    unsigned *order = grouped ? reinterpret_cast<unsigned *>(c + normBytes) : nullptr;
+    uint4 *tiles = tiled ? reinterpret_cast<uint4 *>(c + normBytes + orderBytes) : nullptr;
+    float *BT = reinterpret_cast<float *>(c + normBytes + orderBytes + listBytes);
     hipStream_t st = stream();
-    const unsigned n = pomdp->n;
     if (order)
-        hipLaunchKernelGGL(order_by_action, dim3(1), dim3(1024), 0, st, k, pomdp->m, d_action,
-                           order);
+        hipLaunchKernelGGL(order_by_action, dim3(1), dim3(1024), 0, st, k, m, d_action, order,
+                           tiles, maxTiles);
+    for (unsigned t0 = 0; t0 < maxTiles; t0 += chunkTiles) {
+        const unsigned cnt = std::min(chunkTiles, maxTiles - t0);      // multiples of 8
+        hipLaunchKernelGGL(belief_tiles, dim3(blocks, cnt), dim3(kTileThreads), 0, st, n,
+                           tiles + t0, order, d_rowOf, d_B, BT);
+        if (g_pred.pS16 != nullptr)
+            hipLaunchKernelGGL(belief_update_tiles<unsigned short>, dim3(blocks * cnt),
+                               dim3(kTileThreads), 0, st, n, pomdp->z, blocks, tiles + t0, order,
+                               g_pred.pstart, g_pred.pS16, g_pred.pT, pomdp->d_O, d_observation,
+                               BT, d_Bp);
+        else
+            hipLaunchKernelGGL(belief_update_tiles<int>, dim3(blocks * cnt), dim3(kTileThreads),
+                               0, st, n, pomdp->z, blocks, tiles + t0, order, g_pred.pstart,
+                               g_pred.pS, g_pred.pT, pomdp->d_O, d_observation, BT, d_Bp);
+    }
     const int useLds = n <= (unsigned)kUpdLdsFloats ? 1 : 0;
     const size_t lds = sizeof(float) * ((useLds ? n : 0) + (size_t)kUpdWaves * kUpdScratch);
-    if (g_pred.pS16 != nullptr) {
+    if (tiled) {
+        // done above
+    } else if (g_pred.pS16 != nullptr) {
         hipFuncSetAttribute((const void *)belief_update_batch<unsigned short>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         hipLaunchKernelGGL(belief_update_batch<unsigned short>, dim3(k), dim3(kUB), lds, st, n,
-                           pomdp->m, pomdp->z, g_pred.pstart, g_pred.pS16, g_pred.pT, g_pred.Ot,
+                           m, pomdp->z, g_pred.pstart, g_pred.pS16, g_pred.pT, g_pred.Ot,
                            d_B, d_rowOf, d_action, d_observation, d_Bp, useLds, order);
     } else {
         hipFuncSetAttribute((const void *)belief_update_batch<int>,
                             hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        hipLaunchKernelGGL(belief_update_batch<int>, dim3(k), dim3(kUB), lds, st, n, pomdp->m,
+        hipLaunchKernelGGL(belief_update_batch<int>, dim3(k), dim3(kUB), lds, st, n, m,
                            pomdp->z, g_pred.pstart, g_pred.pS, g_pred.pT, g_pred.Ot, d_B,
                            d_rowOf, d_action, d_observation, d_Bp, useLds, order);
     }

@@ -8,6 +8,8 @@ fp32 (matrix cores): the chosen alpha is the FP64 maximiser except at near-ties 
 bf16 (matrix cores): reported (alpha disagreement rate, value error against FP64); the value
       of the chosen alpha stays within 1e-2 * max |V| of the FP64 maximum.
 """
+import ctypes as ct
+
 import numpy as np
 import pytest
 
@@ -194,6 +196,55 @@ def test_belief_update_batch_bitwise(oracle, n, m, z, ns, k):
     assert np.all(status[:5] == 10)
     print("belief update batch: n=%d k=%d bit-identical (%d impossible observations)"
           % (n, k, int((status == 10).sum())), flush=True)
+
+
+@pytest.mark.parametrize("n,m,z,ns,k", [(1, 2, 3, 1, 4100), (130, 3, 5, 4, 4101),
+                                        (257, 40, 2, 9, 4200), (8192, 2, 3, 3, 33),
+                                        (8200, 3, 2, 4, 70)])
+def test_belief_update_tiles_equal_single_triples(oracle, n, m, z, ns, k):
+    """Batches that go through tiles of 32 triples (many triples, or n from 8,192 on) against the
+    oracle on a sample and against calls below those sizes on every triple: ragged and skewed
+    successor lists, uneven actions, impossible observations, actions and observations out of
+    range (their rows are left as they were)."""
+    import torch
+    from nova_amd import _abi
+    P = synth.pomdp_arrays(n=n, m=m, z=z, ns=min(ns, n), r=2, rz=1, seed=n + k)
+    rng = np.random.default_rng(k)
+    S = P["S"].copy()
+    S[rng.random(S.shape[:2]) < 0.2, -1] = -1
+    S[: n // 2, 0, 0] = 0                      # one state with a long predecessor list
+    P["S"] = S
+    P["O"] = P["O"].copy()
+    P["O"][0, :, 0] = 0.0
+    p = POMDP.from_dict(P)
+    p.initialize_gpu()
+    B = rng.exponential(size=(k, n)).astype(np.float32)
+    B /= B.sum(axis=1, keepdims=True)
+    a = np.minimum(rng.geometric(0.5, k) - 1, m - 1).astype(np.int32)
+    o = rng.integers(0, z, k).astype(np.int32)
+    a[3], o[4] = m, z
+    lib = _abi.load()
+    Bt, at, ot = (torch.from_numpy(x).cuda() for x in (B, a, o))
+
+    def call(lo, hi):
+        out = torch.full((hi - lo, n), -7.0, device="cuda")
+        st = torch.empty(hi - lo, dtype=torch.int32, device="cuda")
+        torch.cuda.synchronize()
+        assert lib.nova_amd_belief_update_batch_gpu(
+            ct.byref(p), hi - lo, Bt[lo:hi].data_ptr(), at[lo:hi].data_ptr(),
+            ot[lo:hi].data_ptr(), out.data_ptr(), st.data_ptr()) == 0
+        return out.cpu().numpy(), st.cpu().numpy()
+
+    got, status = call(0, k)
+    assert status[3] == 1 and status[4] == 1 and np.all(got[3:5] == -7.0)
+    if n < 8192:
+        step = 1000
+        parts = [call(lo, min(lo + step, k)) for lo in range(0, k, step)]
+        assert np.array_equal(bits(got), bits(np.concatenate([x for x, _ in parts])))
+        assert np.array_equal(status, np.concatenate([x for _, x in parts]))
+    for i in [i for i in range(0, k, max(1, k // 40)) if i not in (3, 4)]:
+        rc, bp = oracle.belief_update(P, B[i], int(a[i]), int(o[i]))
+        assert status[i] == rc and np.array_equal(bits(got[i]), bits(bp)), i
 
 
 def bf16_round(x):
