@@ -536,6 +536,241 @@ __global__ __launch_bounds__(kGThreads) void dense_score_bf16(unsigned rows, uns
     }
 }
 
+// ---- single precision on the bf16 matrix cores
+//
+// An fp32 number is the sum of three bf16 numbers, x = h + m + l (8 significant bits each, every
+// one the rounding of what the earlier ones leave), exactly. Of the nine products of two such
+// sums the six largest, hh, hm, mh, hl, lh and mm, differ from the fp32 product by at most about
+// 2^-26 of it, less than its own rounding, and one bf16 matrix instruction sums sixteen of them
+// per fp32 rounding where the fp32 one sums two. Six bf16 products cost 6/16 of the fp32
+// instruction's time. The split is exact for magnitudes in [2^-100, 2^126] and zero; operands
+// with anything else (dense_split_convert reports it: NaN, infinities, values whose parts
+// would overflow or lose bits to underflow) are left to dense_score<float>. The relative error
+// of a row maximum against 64 bits is the smaller here at every size measured: n = 256: 2.0e-7
+// against 2.4e-7, n = 3,000: 6.9e-7 against 7.6e-7, n = 20,000: 1.7e-6 against 2.1e-6 (values
+// within +-3; 1.4e-6 against 2.2e-6 around -20). k = 16,384, r = 4,096, n = 20,000: 20.7 -> 12.1
+// ms a call, the GEMM 11.1 ms: 1.45 PFLOP/s of bf16 products, 0.58 of the peak (0.50 of it in
+// dense_score_bf16, whose LDS reads per matrix instruction are twice as many).
+//
+// Operands lie in the order in which lanes read them from LDS: 1 KB blocks of 32 rows x 16 k,
+// [k / 16][row / 32] with lane 32 c + r's eight k = 8 c .. 8 c + 7 of row r at 16 (32 c + r), per
+// plane (h, m, l), so that copies and LDS reads are linear and free of bank conflicts.
+constexpr int kSplitBlk = 16;                       // k per block and stage
+constexpr int kSplitStages = 3;
+constexpr int kSplitOp = kGT * kSplitBlk * 2;       // one plane of one operand: 8 KB
+constexpr size_t kSplitLdsBytes = (size_t)kSplitStages * 6 * kSplitOp;   // 147,456
+
+// G (float, count / n rows of n) -> the three planes (plane p at GS + p * rowsPad * kpad); rows
+// and columns past the data are zeros. *wild is set to 1 when an element cannot be split
+// exactly. Each lane forms two 16-byte chunks of each plane: 8 consecutive k of one row in two
+// neighbouring k blocks.
+__global__ __launch_bounds__(kGConvThreads) void dense_split_convert(unsigned n, unsigned kpad,
+        size_t count, size_t rowsPad, const float *__restrict__ G, __bf16 *__restrict__ GS,
+        int *__restrict__ wild)
+{
+    const size_t rowsValid = count / n, plane = rowsPad * kpad, chunks = plane / 16;
+    bool bad = false;
+    for (size_t c = blockIdx.x * (size_t)kGConvThreads + threadIdx.x; c < chunks;
+         c += (size_t)gridDim.x * kGConvThreads) {
+        // c: (pair of k blocks, row block, chunk within the block)
+        const size_t kb = c / (rowsPad * 2) * 2, rem = c % (rowsPad * 2);
+        const size_t rowBlk = rem / 64, lane = rem % 64, row = rowBlk * 32 + lane % 32;
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const size_t k0 = (kb + u) * kSplitBlk + lane / 32 * 8;
+            float x[8];
+            if (row < rowsValid && k0 + 8 <= n) {
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+                    x[e] = G[row * n + k0 + e];
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+                    x[e] = (row < rowsValid && k0 + e < n) ? G[row * n + k0 + e] : 0.0f;
+            }
+            bf16x8_t h, m, l;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float ax = fabsf(x[e]);
+                bad = bad || !(ax == 0.0f || (ax >= 0x1p-100f && ax <= 0x1p126f));
+                h[e] = (__bf16)x[e];
+                const float r1 = x[e] - (float)h[e];
+                m[e] = (__bf16)r1;
+                l[e] = (__bf16)(r1 - (float)m[e]);
+            }
+            __bf16 *dst = GS + (((kb + u) * (rowsPad / 32) + rowBlk) * 64 + lane) * 8;
+            *reinterpret_cast<bf16x8_t *>(dst) = h;
+            *reinterpret_cast<bf16x8_t *>(dst + plane) = m;
+            *reinterpret_cast<bf16x8_t *>(dst + 2 * plane) = l;
+        }
+    }
+    if (bad)
+        *wild = 1;
+}
+
+// C = A B^T of split operands with the row argmax of dense_score (one pair): partVal / partJ at
+// jtile * rows + i. 256 x 256 tiles, 8 waves of 128 x 64. Three stages of 16 k lie in LDS. A
+// wave holds a stage's fragments in registers: the smaller planes' are replaced by the next
+// stage's as the products free them, the h fragments alternate between two sets, so LDS reads
+// run behind the 48 matrix instructions of a stage.
+__global__ __launch_bounds__(kGThreads) void dense_score_split(unsigned rows, unsigned cols,
+        unsigned kpad, unsigned rowTiles, unsigned colTiles, const __bf16 *__restrict__ A,
+        const __bf16 *__restrict__ B, float *__restrict__ partVal, int *__restrict__ partJ)
+{
+    extern __shared__ __attribute__((aligned(16))) unsigned char glds[];
+    const unsigned T = rowTiles * colTiles;
+    const unsigned q = (T % 8 == 0) ? (blockIdx.x % 8) * (T / 8) + blockIdx.x / 8 : blockIdx.x;
+    const unsigned groupSize = kGGroup * colTiles, firstRow = (q / groupSize) * kGGroup;
+    const unsigned rowsHere = min(kGGroup, rowTiles - firstRow), inGroup = q % groupSize;
+    const unsigned itile = firstRow + inGroup % rowsHere, jtile = inGroup / rowsHere;
+    const unsigned i0 = itile * kGT, j0 = jtile * kGT;
+    const unsigned t = threadIdx.x, l = t % 64, w = __builtin_amdgcn_readfirstlane(t / 64);
+    const unsigned wr = w / 4, wc = w % 4;
+    const size_t aRows = (size_t)rowTiles * kGT, bRows = (size_t)colTiles * kGT;
+    const size_t aPlane = aRows * kpad, bPlane = bRows * kpad;
+    // wave w copies row block w of each plane: six 1 KB blocks a stage
+    const __bf16 *As = A + (size_t)(i0 / 32 + w) * 512 + l * 8;
+    const __bf16 *Bs = B + (size_t)(j0 / 32 + w) * 512 + l * 8;
+    auto issue = [&](unsigned s) {
+        unsigned char *st = glds + (size_t)(s % kSplitStages) * 6 * kSplitOp + w * 1024;
+        const __bf16 *as = As + (size_t)s * aRows * kSplitBlk;
+        const __bf16 *bs = Bs + (size_t)s * bRows * kSplitBlk;
+#pragma unroll
+        for (int p = 0; p < 3; p++) {
+            __builtin_amdgcn_global_load_lds((const void *)(as + p * aPlane),
+                                             (void *)(st + p * kSplitOp), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((const void *)(bs + p * bPlane),
+                                             (void *)(st + (3 + p) * kSplitOp), 16, 0, 0);
+        }
+    };
+    const unsigned aAddr = wr * 4096 + l * 16, bAddr = 3 * kSplitOp + wc * 2048 + l * 16;
+
+    floatx16_t acc[4][2];
+#pragma unroll
+    for (int x = 0; x < 4; x++)
+#pragma unroll
+        for (int y = 0; y < 2; y++)
+#pragma unroll
+            for (int v = 0; v < 16; v++)
+                acc[x][y][v] = 0.0f;
+    auto readA = [&](const unsigned char *st, int p, bf16x8_t (&f)[4]) {
+#pragma unroll
+        for (int x = 0; x < 4; x++)
+            f[x] = *reinterpret_cast<const bf16x8_t *>(st + p * kSplitOp + aAddr + x * 1024);
+    };
+    auto readB = [&](const unsigned char *st, int p, bf16x8_t (&f)[2]) {
+#pragma unroll
+        for (int y = 0; y < 2; y++)
+            f[y] = *reinterpret_cast<const bf16x8_t *>(st + p * kSplitOp + bAddr + y * 1024);
+    };
+    auto mul = [&](const bf16x8_t (&fa)[4], const bf16x8_t (&fb)[2]) {
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            acc[i / 2][i % 2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i / 2], fb[i % 2],
+                                                                      acc[i / 2][i % 2], 0, 0, 0);
+    };
+    const unsigned nk = kpad / kSplitBlk;           // a multiple of 4
+    issue(0);
+    issue(1);
+    issue(2);
+    wait_vmem<12>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    bf16x8_t ah[2][4], am[4], al[4], bh[2][2], bm[2], bl[2];
+    readA(glds, 2, al);
+    readB(glds, 0, bh[0]);
+    readA(glds, 1, am);
+    readB(glds, 1, bm);
+    readA(glds, 0, ah[0]);
+    readB(glds, 2, bl);
+    // stage ks: its fragments are in registers; MORE: stage ks + 1 is there to be read
+    auto stage = [&](unsigned ks, int cur, bool more) {
+        mul(al, bh[cur]);
+        const unsigned char *st = glds + (size_t)((ks + 1) % kSplitStages) * 6 * kSplitOp;
+        if (more) {
+            // stage ks + 1 landed (only stage ks + 2's six copies may be outstanding); past the
+            // barrier every wave holds stage ks in registers, so its buffer is refilled
+            if (ks + 2 < nk)
+                asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)" ::: "memory");
+            else
+                asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            if (ks + 3 < nk)
+                issue(ks + 3);
+            readA(st, 2, al);
+            readB(st, 0, bh[cur ^ 1]);
+        }
+        mul(am, bm);
+        mul(am, bh[cur]);
+        if (more) {
+            readA(st, 1, am);
+            readA(st, 0, ah[cur ^ 1]);
+        }
+        mul(ah[cur], bl);
+        if (more)
+            readB(st, 2, bl);
+        mul(ah[cur], bm);
+        if (more)
+            readB(st, 1, bm);
+        mul(ah[cur], bh[cur]);
+    };
+    for (unsigned ks = 0; ks + 2 < nk; ks += 2) {
+        stage(ks, 0, true);
+        stage(ks + 1, 1, true);
+    }
+    stage(nk - 2, 0, true);
+    stage(nk - 1, 1, false);
+    __syncthreads();
+
+    // epilogue: per row, the first maximiser over this tile's 256 columns
+    float *redV = reinterpret_cast<float *>(glds);             // [4][256]
+    int *redJ = reinterpret_cast<int *>(glds + 4 * kGT * sizeof(float));
+#pragma unroll
+    for (int x = 0; x < 4; x++) {
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+            float bv = kLow;
+            int bj = INT_MAX;
+#pragma unroll
+            for (int y = 0; y < 2; y++) {
+                const unsigned j = j0 + wc * 64 + y * 32 + l % 32;
+                const float val = acc[x][y][v];
+                if (j < cols && better(val, (int)j, bv, bj)) {
+                    bv = val;
+                    bj = (int)j;
+                }
+            }
+            for (int o2 = 16; o2 >= 1; o2 >>= 1) {
+                const float ov = __shfl_xor(bv, o2, 32);
+                const int oj = __shfl_xor(bj, o2, 32);
+                if (better(ov, oj, bv, bj)) {
+                    bv = ov;
+                    bj = oj;
+                }
+            }
+            if (l % 32 == 0) {
+                const unsigned row = wr * 128 + x * 32 + (v % 4) + 4 * (l / 32) + 8 * (v / 4);
+                redV[wc * kGT + row] = bv;
+                redJ[wc * kGT + row] = bj;
+            }
+        }
+    }
+    __syncthreads();
+    if (t < kGT && i0 + t < rows) {
+        float v0 = redV[t];
+        int jv = redJ[t];
+#pragma unroll
+        for (int q2 = 1; q2 < 4; q2++)
+            if (better(redV[q2 * kGT + t], redJ[q2 * kGT + t], v0, jv)) {
+                v0 = redV[q2 * kGT + t];
+                jv = redJ[q2 * kGT + t];
+            }
+        partVal[(size_t)jtile * rows + i0 + t] = v0;
+        partJ[(size_t)jtile * rows + i0 + t] = jv;
+    }
+}
+
 // The bf16 reference path (dense_score<__bf16> on row-major operands) instead of
 // dense_score_bf16, for comparisons: NOVA_AMD_DENSE_KERNEL=legacy.
 inline bool dense_legacy_bf16()

@@ -7,8 +7,9 @@
 //              separately, as the reference: V and the action equal nova's bit for bit. A
 //              vector-ALU tile kernel: 64 beliefs x 64 alphas per workgroup, each lane a 4 x 4
 //              block, both operands staged state-major in LDS 32 states at a time.
-//      fp32  - the dense GEMM of dense_gemm.h on the matrix cores (v_mfma_f32_32x32x2_f32):
-//              fp32 products, fp32 sums in the matrix cores' order.
+//      fp32  - the split GEMM of dense_gemm.h on the bf16 matrix cores (three bf16 parts of
+//              each operand, six products, fp32 sums), its fp32 GEMM (v_mfma_f32_32x32x2_f32)
+//              where the operands have no such parts.
 //      bf16  - dense_score_bf16 of dense_gemm.h: bf16 operands in the k-blocked layout,
 //              copied straight into LDS, fp32 accumulation (v_mfma_f32_32x32x16_bf16): about
 //              3 significant digits per operand.
@@ -167,7 +168,9 @@ __global__ __launch_bounds__(256) void alpha_value_merge(unsigned k, unsigned ti
 // accesses. VEC: rows 16-byte aligned (n % 4 == 0).
 constexpr unsigned kFewAlphas = 16;
 
-template <int X, int CH, bool VEC>
+// PREC: the call's precision, 0 exact, 1 fp32 (each product and sum rounded once, by an FMA), 2
+// operands rounded to bf16 on the way into LDS and fp32 sums.
+template <int X, int CH, bool VEC, int PREC>
 __global__ __launch_bounds__(64) void alpha_value_few(unsigned k, unsigned n, unsigned r,
         const float *__restrict__ B, const float *__restrict__ G, float *__restrict__ partV,
         int *__restrict__ partJ)
@@ -211,11 +214,12 @@ __global__ __launch_bounds__(64) void alpha_value_few(unsigned k, unsigned n, un
 #pragma unroll
         for (int u = 0; u < kPer; u++) {
             const unsigned e = u * 64 + lane;
+            auto in = [](float v) { return PREC == 2 ? (float)(__bf16)v : v; };
             if constexpr (VEC)
                 *reinterpret_cast<float4 *>(&buf[e / kAcross * kStride + e % kAcross * 4]) =
-                    pre4[u];
+                    make_float4(in(pre4[u].x), in(pre4[u].y), in(pre4[u].z), in(pre4[u].w));
             else
-                buf[e / kAcross * kStride + e % kAcross] = pre[u];
+                buf[e / kAcross * kStride + e % kAcross] = in(pre[u]);
         }
         __syncthreads();
         if (s0 + CH < n)
@@ -244,7 +248,8 @@ __global__ __launch_bounds__(64) void alpha_value_few(unsigned k, unsigned n, un
 #pragma unroll
                     for (int x = 0; x < X; x++) {
                         const float b4[4] = {bq[x][v].x, bq[x][v].y, bq[x][v].z, bq[x][v].w};
-                        acc[x] = __fadd_rn(acc[x], __fmul_rn(g4[e], b4[e]));
+                        acc[x] = PREC == 0 ? __fadd_rn(acc[x], __fmul_rn(g4[e], b4[e]))
+                                           : __fmaf_rn(g4[e], b4[e], acc[x]);
                     }
             }
         };
@@ -324,7 +329,7 @@ __global__ __launch_bounds__(64) void alpha_value_merge_few(unsigned k, unsigned
         jOut[i] = none ? -1 : bj;
 }
 
-template <int X, int CH>
+template <int X, int CH, int PREC>
 void launch_few(unsigned k, unsigned n, unsigned r, const float *B, const float *G, float *partV,
                 int *partJ, hipStream_t st)
 {
@@ -332,33 +337,45 @@ void launch_few(unsigned k, unsigned n, unsigned r, const float *B, const float 
                                      reinterpret_cast<uintptr_t>(G)) & 15u) == 0;
     const dim3 g((k + 4 * X - 1) / (4 * X), (r + kFewAlphas - 1) / kFewAlphas);
     if (vec)
-        hipLaunchKernelGGL((alpha_value_few<X, CH, true>), g, dim3(64), 0, st, k, n, r, B, G,
-                           partV, partJ);
+        hipLaunchKernelGGL((alpha_value_few<X, CH, true, PREC>), g, dim3(64), 0, st, k, n, r, B,
+                           G, partV, partJ);
     else
-        hipLaunchKernelGGL((alpha_value_few<X, CH, false>), g, dim3(64), 0, st, k, n, r, B, G,
-                           partV, partJ);
+        hipLaunchKernelGGL((alpha_value_few<X, CH, false, PREC>), g, dim3(64), 0, st, k, n, r, B,
+                           G, partV, partJ);
 }
 
-// Beliefs per lane of alpha_value_few for a call, or 0 where alpha_value_exact is the faster:
-// one while that gives at most 2,048 waves (two per SIMD), then two, until alpha_value_exact has
+template <int PREC>
+void launch_few_of(unsigned few, unsigned k, unsigned n, unsigned r, const float *B,
+                   const float *G, float *partV, int *partJ, hipStream_t st)
+{
+    if (few == 1)
+        launch_few<1, 256, PREC>(k, n, r, B, G, partV, partJ, st);
+    else
+        launch_few<2, 128, PREC>(k, n, r, B, G, partV, partJ, st);
+}
+
+// Beliefs per lane of alpha_value_few for a call, or 0 where the mode's own kernel is the faster:
+// one while that gives at most 1,024 waves (one per SIMD), then two, until alpha_value_exact has
 // a workgroup per CU and more. us of a call, 0 / 1 / 2 beliefs per lane: n = 5,000, r = 1,024:
 // k = 4: 602 / 62 / 90; k = 256: 630 / 208 / 131; k = 2,048: 595 / 1,189 / 745. n = 20,000,
 // r = 4,096: k = 1: 2,400 / 204 / 311; k = 64: 2,480 / 829 / 460; k = 256: 2,470 / 2,490 /
 // 1,540; k = 512: 2,290 / 4,660 / 3,150.
 constexpr size_t kFewPairs = 5u << 18;       // most (belief, alpha) pairs, 1.25 Mi
 
-unsigned few_beliefs(unsigned k, unsigned r)
+unsigned few_beliefs(unsigned k, unsigned r, int precision)
 {
-    if ((size_t)k * r > kFewPairs || r > 65535u * kFewAlphas)   // (the grid's y extent)
+    if ((size_t)k * r > kFewPairs || r > 65535u * kFewAlphas ||       // (the grid's y extent)
+            precision != 0)
         return 0;
     const size_t waves = (size_t)((k + 3) / 4) * ((r + kFewAlphas - 1) / kFewAlphas);
-    return waves <= 2048 ? 1 : 2;
+    return waves <= 1024 ? 1 : 2;
 }
 
 // Alphas per partial of the exact mode.
 inline unsigned exact_tile(unsigned few) { return few ? kFewAlphas : (unsigned)kVT; }
 
-void launch_exact(unsigned few, unsigned k, unsigned n, unsigned r, const float *B,
+// Partials and merge on the vector ALUs: the exact mode, and the others' calls of few beliefs.
+void launch_exact(unsigned few, int precision, unsigned k, unsigned n, unsigned r, const float *B,
                   const float *G, const unsigned *pi, float *partV, int *partJ, float *V,
                   unsigned *act, int *jOut, hipStream_t st)
 {
@@ -370,10 +387,12 @@ void launch_exact(unsigned few, unsigned k, unsigned n, unsigned r, const float 
                            partV, partJ, pi, V, act, jOut);
         return;
     }
-    if (few == 1)
-        launch_few<1, 256>(k, n, r, B, G, partV, partJ, st);
+    if (precision == 0)
+        launch_few_of<0>(few, k, n, r, B, G, partV, partJ, st);
+    else if (precision == 1)
+        launch_few_of<1>(few, k, n, r, B, G, partV, partJ, st);
     else
-        launch_few<2, 128>(k, n, r, B, G, partV, partJ, st);
+        launch_few_of<2>(few, k, n, r, B, G, partV, partJ, st);
     hipLaunchKernelGGL(alpha_value_merge_few, dim3(k), dim3(64), 0, st, k, tiles, partV, partJ,
                        pi, V, act, jOut);
 }
@@ -1037,6 +1056,66 @@ int belief_update_rows(const nova::POMDP *pomdp, unsigned k, const float *d_B,
     return NOVA_SUCCESS;
 }
 
+// The fp32 mode on the bf16 matrix cores (dense_score_split). *done stays false when the
+// operands cannot be split exactly or its workspace does not fit: the fp32 instructions do the
+// call then.
+static int value_split(unsigned n, unsigned r, const float *d_Gamma, const unsigned *d_pi,
+                       unsigned k, const float *d_B, float *d_V, unsigned *d_action,
+                       int *d_alpha, const char *fn, bool *done)
+{
+    hipStream_t st = stream();
+    const unsigned rowTiles = (k + kGT - 1) / kGT, colTiles = (r + kGT - 1) / kGT;
+    const unsigned kpad = (n + kGKPad - 1) / kGKPad * kGKPad;
+    const size_t aRows = (size_t)rowTiles * kGT, gRows = (size_t)colTiles * kGT;
+    const size_t bPart = up256((size_t)colTiles * k * sizeof(float));
+    const size_t bA = up256(3 * aRows * kpad * sizeof(__bf16));
+    const size_t bG = up256(3 * gRows * kpad * sizeof(__bf16));
+    void *mem = nullptr;
+    size_t freeBytes = 0, totalBytes = 0;
+    const size_t bytes = 256 + 2 * bPart + bA + bG;
+    if (g_valueArena.mem == nullptr || g_valueArena.bytes < bytes)
+        if (hipMemGetInfo(&freeBytes, &totalBytes) != hipSuccess ||
+                freeBytes + g_valueArena.bytes < bytes + ((size_t)64 << 20))
+            return NOVA_SUCCESS;
+    int rc = arena_get(g_valueArena, bytes, fn, mem);
+    if (rc != NOVA_SUCCESS)
+        return rc;
+    g_valueShape = DenseShape();      // the fp32 layout's padding is overwritten
+    char *c = static_cast<char *>(mem);
+    int *wild = reinterpret_cast<int *>(c);
+    float *partV = reinterpret_cast<float *>(c + 256);
+    int *partJ = reinterpret_cast<int *>(c + 256 + bPart);
+    __bf16 *A = reinterpret_cast<__bf16 *>(c + 256 + 2 * bPart);
+    __bf16 *G = reinterpret_cast<__bf16 *>(c + 256 + 2 * bPart + bA);
+    hipFuncSetAttribute((const void *)dense_score_split,
+                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSplitLdsBytes);
+    const auto blocks = [&](size_t rowsPad) {
+        return dim3((unsigned)std::min<size_t>(
+            (rowsPad * kpad / 16 + kGConvThreads - 1) / kGConvThreads, 65536));
+    };
+    hipError_t e = hipMemsetAsync(wild, 0, sizeof(int), st);
+    hipLaunchKernelGGL(dense_split_convert, blocks(aRows), dim3(kGConvThreads), 0, st, n, kpad,
+                       (size_t)k * n, aRows, d_B, A, wild);
+    hipLaunchKernelGGL(dense_split_convert, blocks(gRows), dim3(kGConvThreads), 0, st, n, kpad,
+                       (size_t)r * n, gRows, d_Gamma, G, wild);
+    hipLaunchKernelGGL(dense_score_split, dim3(rowTiles * colTiles), dim3(kGThreads),
+                       kSplitLdsBytes, st, k, r, kpad, rowTiles, colTiles,
+                       (const __bf16 *)A, (const __bf16 *)G, partV, partJ);
+    hipLaunchKernelGGL(alpha_value_merge, dim3((k + 255) / 256), dim3(256), 0, st, k, colTiles,
+                       partV, partJ, d_pi, d_V, d_action, d_alpha);
+    if (e == hipSuccess)
+        e = hipGetLastError();
+    int flag = 0;
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(&flag, wild, sizeof(int), hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess)
+        e = hipStreamSynchronize(st);
+    if (e != hipSuccess)
+        return hip_fail(e, fn, "Kernel execution failed.", NOVA_ERROR_KERNEL_EXECUTION);
+    *done = flag == 0;
+    return NOVA_SUCCESS;
+}
+
 } // namespace nova_amd
 
 using namespace nova_amd;
@@ -1056,8 +1135,8 @@ extern "C" int nova_amd_alpha_vectors_value_and_action_gpu(unsigned int n, unsig
     }
     std::lock_guard<std::mutex> lock(g_valueMutex);
     hipStream_t st = stream();
-    const bool exact = precision == 0;
-    const unsigned few = exact ? few_beliefs(k, r) : 0;
+    const unsigned few = few_beliefs(k, r, precision);
+    const bool exact = precision == 0 || few != 0;       // on the vector ALUs
     const unsigned tileW = exact ? exact_tile(few) : (unsigned)kGT;
     const unsigned colTiles = (r + tileW - 1) / tileW;
     const unsigned rowTiles = (k + kGT - 1) / kGT;
@@ -1066,13 +1145,19 @@ extern "C" int nova_amd_alpha_vectors_value_and_action_gpu(unsigned int n, unsig
     const size_t bPart = up256((size_t)colTiles * k * sizeof(float));
     size_t bytes = 2 * bPart;
     size_t bA = 0, bG = 0, bS = 0;
+    void *mem = nullptr;
+    if (!exact && precision == 1) {
+        bool done = false;
+        const int rcs = value_split(n, r, d_Gamma, d_pi, k, d_B, d_V, d_action, d_alpha, fn, &done);
+        if (rcs != NOVA_SUCCESS || done)
+            return rcs;
+    }
     if (!exact) {
         bA = up256((size_t)rowTiles * kGT * kpad * inSize);
         bG = up256((size_t)colTiles * kGT * kpad * inSize);
         bS = up256(sizeof(float) * kpad);
         bytes += bA + bG + bS;
     }
-    void *mem = nullptr;
     int rc = arena_get(g_valueArena, bytes, fn, mem);
     if (rc != NOVA_SUCCESS)
         return rc;
@@ -1082,7 +1167,8 @@ extern "C" int nova_amd_alpha_vectors_value_and_action_gpu(unsigned int n, unsig
     hipError_t e = hipSuccess;
     if (exact) {
         g_valueShape = DenseShape();   // the partials may overwrite the dense operands' padding
-        launch_exact(few, k, n, r, d_B, d_Gamma, d_pi, partV, partJ, d_V, d_action, d_alpha, st);
+        launch_exact(few, precision, k, n, r, d_B, d_Gamma, d_pi, partV, partJ, d_V, d_action,
+                     d_alpha, st);
     } else {
         void *A = c + 2 * bPart, *Gi = c + 2 * bPart + bA;
         float *ones = reinterpret_cast<float *>(c + 2 * bPart + bA + bG);
@@ -1243,7 +1329,7 @@ extern "C" int nova_amd_alpha_vectors_value_and_action_noalloc_gpu(unsigned int 
     if (c == nullptr)
         return NOVA_ERROR_KERNEL_EXECUTION;
     // the narrower tiles of few beliefs have four times the partials: only where they fit too
-    unsigned few = few_beliefs(k, r);
+    unsigned few = few_beliefs(k, r, 0);
     if (few) {
         colTiles = (r + kFewAlphas - 1) / kFewAlphas;
         if (2 * up256(colTiles * k * sizeof(float)) <= kNoAllocScratchBytes)
@@ -1254,7 +1340,7 @@ extern "C" int nova_amd_alpha_vectors_value_and_action_noalloc_gpu(unsigned int 
     hipStream_t st = stream();
     float *partV = reinterpret_cast<float *>(c);
     int *partJ = reinterpret_cast<int *>(c + bPart);
-    launch_exact(few, k, n, r, d_B, d_Gamma, d_pi, partV, partJ, d_V, d_action, d_alpha, st);
+    launch_exact(few, 0, k, n, r, d_B, d_Gamma, d_pi, partV, partJ, d_V, d_action, d_alpha, st);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess)
         e = hipStreamSynchronize(st);

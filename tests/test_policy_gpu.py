@@ -149,6 +149,49 @@ def test_bf16_matrix_cores_reported(k, n, r):
     assert err <= 1e-2 and np.array_equal(act, pi[j])
 
 
+# more than 1.25 Mi (belief, alpha) pairs: the split GEMM
+@pytest.mark.parametrize("k,n,r", [(1300, 1, 1100), (1025, 64, 1300), (5200, 130, 257),
+                                   (700, 1000, 2000)])
+def test_fp32_split_vs_fp64(k, n, r):
+    """fp32 as three bf16 parts: V within n fp32 roundings of the FP64 maximum, over operands of
+    mixed signs and magnitudes (2^-100 and 2^60 among them)."""
+    rng = np.random.default_rng(k + n)
+    G = rng.standard_normal((r, n)).astype(np.float32) * \
+        np.float32(2.0) ** rng.integers(-12, 13, (r, n)).astype(np.float32)
+    B = rng.standard_normal((k, n)).astype(np.float32)
+    B[rng.random((k, n)) < 0.3] = 0.0
+    G[0, 0], B[1, 0] = 2.0 ** -100, 2.0 ** 60
+    pi = rng.integers(0, 5, r).astype(np.uint32)
+    V, act, j = policy(G, pi).value_and_action_batch(B, "fp32", return_alpha=True)
+    V, act, j = V.cpu().numpy(), act.cpu().numpy(), j.cpu().numpy()
+    C = B.astype(np.float64) @ G.astype(np.float64).T
+    bound = (n + 1) * 2.0 ** -24 * (np.abs(B).astype(np.float64) @ np.abs(G).T).max(axis=1)
+    assert np.all(np.abs(V - C.max(axis=1)) <= bound)
+    assert np.all(C.max(axis=1) - C[np.arange(k), j] <= 2 * bound)
+    assert np.array_equal(act, pi[j])
+
+
+@pytest.mark.parametrize("odd", [np.inf, -np.inf, np.nan, 3.4e38, 1e-36, 1e-40])
+def test_fp32_operands_without_bf16_parts(odd):
+    """One operand value that has no exact bf16 parts: the call is left to the fp32 matrix
+    instructions, and gives what they give (an infinity wins, a NaN never does)."""
+    k, n, r = 1400, 70, 1000
+    G, pi, B = instance(k, n, r, seed=3)
+    B[:, 5] = 0.0
+    B[7, 5] = 0.5
+    G[11, 5] = odd
+    with np.errstate(invalid="ignore"):
+        C = B.astype(np.float64) @ G.astype(np.float64).T
+    C[np.isnan(C)] = -np.inf
+    V, act, j = policy(G, pi).value_and_action_batch(B, "fp32", return_alpha=True)
+    V, j = V.cpu().numpy().astype(np.float64), j.cpu().numpy()
+    best = C.max(axis=1)
+    fine = np.isfinite(best)
+    assert np.allclose(V[fine], best[fine], rtol=1e-5, atol=1e-5)
+    assert np.array_equal(V[~fine], best[~fine])
+    assert np.all(j[~fine] == 11)
+
+
 def test_large_fp32_against_exact_sample():
     """At n = 20,000 and r = 4,096 (the dense PBVI size) with k = 8,192 beliefs: fp32 against
     exact on the first 256 beliefs (same choice or a near-tie)."""
