@@ -13,6 +13,7 @@
 //      bf16  - dense_score_bf16 of dense_gemm.h: bf16 operands in the k-blocked layout,
 //              copied straight into LDS, fp32 accumulation (v_mfma_f32_32x32x16_bf16): about
 //              3 significant digits per operand.
+//    Calls of few beliefs run on the vector ALUs in every mode (alpha_value_few).
 //    All modes write per-(belief, alpha tile) maxima that one merge kernel reduces in tile
 //    order (the earlier tile wins ties, i.e. the first maximiser overall).
 // 2. Belief updates of k (belief, action, observation) triples
@@ -359,13 +360,18 @@ void launch_few_of(unsigned few, unsigned k, unsigned n, unsigned r, const float
 // a workgroup per CU and more. us of a call, 0 / 1 / 2 beliefs per lane: n = 5,000, r = 1,024:
 // k = 4: 602 / 62 / 90; k = 256: 630 / 208 / 131; k = 2,048: 595 / 1,189 / 745. n = 20,000,
 // r = 4,096: k = 1: 2,400 / 204 / 311; k = 64: 2,480 / 829 / 460; k = 256: 2,470 / 2,490 /
-// 1,540; k = 512: 2,290 / 4,660 / 3,150.
+// 1,540; k = 512: 2,290 / 4,660 / 3,150. The same line serves fp32, whose GEMM has a workgroup
+// per 256 x 256 block of C (us, the fp32 GEMM / the split GEMM / this: n = 20,000, r = 4,096,
+// k = 16: 5,140 / 2,310 / 214; k = 256: 5,150 / 2,320 / 1,510; n = 1,000, r = 200, k = 4,096:
+// 315 / 177 / 82). bf16 calls take it up to kFewBf16 beliefs (n = 20,000, r = 4,096: k = 8: 213,
+// k = 64: 408 against 508 of the bf16 GEMM at any k up to 256).
 constexpr size_t kFewPairs = 5u << 18;       // most (belief, alpha) pairs, 1.25 Mi
+constexpr unsigned kFewBf16 = 64;
 
 unsigned few_beliefs(unsigned k, unsigned r, int precision)
 {
     if ((size_t)k * r > kFewPairs || r > 65535u * kFewAlphas ||       // (the grid's y extent)
-            precision != 0)
+            (precision == 2 && (k > kFewBf16 || dense_legacy_bf16())))
         return 0;
     const size_t waves = (size_t)((k + 3) / 4) * ((r + kFewAlphas - 1) / kFewAlphas);
     return waves <= 1024 ? 1 : 2;

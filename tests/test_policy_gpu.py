@@ -149,6 +149,26 @@ def test_bf16_matrix_cores_reported(k, n, r):
     assert err <= 1e-2 and np.array_equal(act, pi[j])
 
 
+@pytest.mark.parametrize("k,n,r", [(1, 1, 1), (5, 17, 16), (9, 257, 33), (64, 130, 300),
+                                   (300, 40, 4000)])
+@pytest.mark.parametrize("prec", ["fp32", "bf16"])
+def test_few_beliefs_fp32_and_bf16(k, n, r, prec):
+    """Calls of few beliefs on the vector ALUs: V within the accumulation error of n fp32 sums
+    (n * 2^-24 * max sum |b||alpha|) of the FP64 maximum over the operands as the mode rounds
+    them, and the chosen alpha's value too."""
+    G, pi, B = instance(k, n, r, seed=13 * k + n + r)
+    p = policy(G, pi)
+    V, act, j = p.value_and_action_batch(B, prec, return_alpha=True)
+    V, act, j = V.cpu().numpy(), act.cpu().numpy(), j.cpu().numpy()
+    if prec == "bf16":
+        G, B = bf16_round(G), bf16_round(B)
+    C = B.astype(np.float64) @ G.astype(np.float64).T
+    bound = (n + 1) * 2.0 ** -24 * (np.abs(B).astype(np.float64) @ np.abs(G).T).max(axis=1) + 1e-30
+    assert np.all(np.abs(V - C.max(axis=1)) <= bound)
+    assert np.all(C.max(axis=1) - C[np.arange(k), j] <= 2 * bound)
+    assert np.array_equal(act, pi[j])
+
+
 # more than 1.25 Mi (belief, alpha) pairs: the split GEMM
 @pytest.mark.parametrize("k,n,r", [(1300, 1, 1100), (1025, 64, 1300), (5200, 130, 257),
                                    (700, 1000, 2000)])
