@@ -273,9 +273,20 @@ __device__ void build_support(SupportLds &L, unsigned i, unsigned a, unsigned m,
         if (t < 64) {
             int c = 0;
             if ((int)t < kEnd) {
+                // the valid prefix, four successors requested together
                 const size_t row = ((size_t)L.sK[t] * m + a) * ns;
-                while (c < (int)ns && S[row + c] >= 0)
-                    c++;
+                bool end = false;
+                for (unsigned c0 = 0; c0 < ns && !end; c0 += 4) {
+                    int sp[4];
+#pragma unroll
+                    for (unsigned e = 0; e < 4; e++)
+                        sp[e] = S[row + min(c0 + e, ns - 1)];
+#pragma unroll
+                    for (unsigned e = 0; e < 4; e++) {
+                        end = end || c0 + e >= ns || sp[e] < 0;
+                        c += end ? 0 : 1;
+                    }
+                }
             }
             for (int off = 1; off < 64; off <<= 1) {
                 const int y = __shfl_up(c, off);
@@ -1730,6 +1741,72 @@ __device__ __forceinline__ void fused_stage_copy(T *dst, F get, unsigned count, 
     }
 }
 
+// The scores of every (observation, alpha): lane t takes alpha t mod jl (jl a power of two) and Q
+// observations at a time, kPB / jl apart, so one read of Gamma serves Q sums. The support's
+// pairs are the same for every lane; four of them are read together, then their Gamma and O*T
+// values, then their sums follow in the reference's order. At one wave per SIMD the chains of
+// LDS reads were the iteration's time.
+template <int Q>
+__device__ __forceinline__ void fused_scores(const SupportLds &L, const float *ota,
+        const float *G, float *sc, unsigned n, unsigned ns, unsigned z, unsigned r, unsigned gs,
+        unsigned jl, float gamma)
+{
+    const unsigned groups = kPB / jl, og = threadIdx.x / jl, plane = n * ns;
+    const int kEnd = __builtin_amdgcn_readfirstlane(L.kEnd);
+    for (unsigned j0 = threadIdx.x % jl; j0 < r; j0 += jl) {
+        const float *Gj = G + (size_t)j0 * gs;
+        for (unsigned o0 = og; o0 < z; o0 += Q * groups) {
+            const float *ot[Q];
+            float value[Q];
+#pragma unroll
+            for (int q = 0; q < Q; q++) {
+                ot[q] = ota + (size_t)min(o0 + q * groups, z - 1) * plane;
+                value[q] = 0.0f;
+            }
+            int u1 = __builtin_amdgcn_readfirstlane(L.startK[0]);
+            for (int k = 0; k < kEnd; k++) {
+                const int first = u1;
+                u1 = __builtin_amdgcn_readfirstlane(L.startK[k + 1]);
+                const float bk = L.bK[k];
+                float vt[Q];
+#pragma unroll
+                for (int q = 0; q < Q; q++)
+                    vt[q] = 0.0f;
+                for (int u0 = first; u0 < u1; u0 += 4) {
+                    int sp[4], ou[4];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        sp[e] = L.spU[min(u0 + e, u1 - 1)];
+                        ou[e] = L.otU[min(u0 + e, u1 - 1)];
+                    }
+                    float g[4], w[Q][4];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        g[e] = Gj[sp[e]];
+#pragma unroll
+                        for (int q = 0; q < Q; q++)
+                            w[q][e] = ot[q][ou[e]];
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        if (u0 + e < u1) {
+#pragma unroll
+                            for (int q = 0; q < Q; q++)
+                                vt[q] = __fadd_rn(vt[q], __fmul_rn(w[q][e], g[e]));
+                        }
+                }
+#pragma unroll
+                for (int q = 0; q < Q; q++)
+                    value[q] = __fadd_rn(value[q], __fmul_rn(__fmul_rn(vt[q], gamma), bk));
+            }
+#pragma unroll
+            for (int q = 0; q < Q; q++)
+                if (o0 + q * groups < z)
+                    sc[(o0 + q * groups) * r + j0] = value[q];
+        }
+    }
+}
+
 __global__ __launch_bounds__(kPB) void pbvi_fused(const PbviInst *__restrict__ insts,
         const unsigned *__restrict__ off, unsigned count, unsigned iter, unsigned flip)
 {
@@ -1799,18 +1876,15 @@ __global__ __launch_bounds__(kPB) void pbvi_fused(const PbviInst *__restrict__ i
         build_support(L, 0, 0, 1, ns, rz, Sa, Zi, Bi, scratch);   // ends with a barrier
         const int kEnd = L.kEnd;
         // score of alpha j under observation o: sum_k ((sum_l (O*T) * Gamma[j, sp]) * gamma) * b_k
-        for (unsigned x = t; x < z * r; x += kPB) {
-            const unsigned o = x / r, j = x % r;
-            const float *ot = ota + (size_t)o * n * ns;
-            const float *Gj = G + (size_t)j * gs;
-            float value = 0.0f;
-            for (int k = 0; k < kEnd; k++) {
-                float vt = 0.0f;
-                for (int u = L.startK[k]; u < L.startK[k + 1]; u++)
-                    vt = __fadd_rn(vt, __fmul_rn(ot[L.otU[u]], Gj[L.spU[u]]));
-                value = __fadd_rn(value, __fmul_rn(__fmul_rn(vt, gamma), L.bK[k]));
-            }
-            sc[x] = value;
+        {
+            const unsigned jl = min((unsigned)kPB, 1u << (32 - __clz((int)max(r, 2u) - 1)));
+            const unsigned groups = kPB / jl;
+            if (z <= groups)
+                fused_scores<1>(L, ota, G, sc, n, ns, z, r, gs, jl, gamma);
+            else if (z <= 2 * groups)
+                fused_scores<2>(L, ota, G, sc, n, ns, z, r, gs, jl, gamma);
+            else
+                fused_scores<4>(L, ota, G, sc, n, ns, z, r, gs, jl, gamma);
         }
         __syncthreads();
         // first maximiser per observation by strict '>' from -1e10 (none: alpha 0): 32 lanes
@@ -1841,31 +1915,69 @@ __global__ __launch_bounds__(kPB) void pbvi_fused(const PbviInst *__restrict__ i
             }
         }
         __syncthreads();
-        // alpha(s) = R[s,a] + sum_o (gamma * sum_l (O*T) * Gamma[j*_o, sp]), o ascending
-        for (unsigned s = t; s < n; s += kPB) {
+        // alpha(s) = R[s,a] + sum_o (gamma * sum_l (O*T) * Gamma[j*_o, sp]), o ascending: the inner
+        // sums of every (observation, state) in parallel into the scores' LDS where they fit
+        // there, then each state adds its terms in order
+        auto inner = [&](unsigned o, unsigned s) {
             const int *rw = Sa + (size_t)s * ns;
-            float al = Rall[(size_t)s * m + a];
-            for (unsigned o = 0; o < z; o++) {
-                const float *Gj = G + (size_t)js[o] * gs;
-                const float *ot = ota + ((size_t)o * n + s) * ns;
-                float vt = 0.0f;
-                for (unsigned l = 0; l < ns; l++) {
-                    const int sp = rw[l];
-                    if (sp < 0)
-                        break;
-                    vt = __fadd_rn(vt, __fmul_rn(ot[l], Gj[sp]));
+            const float *Gj = G + (size_t)js[o] * gs;
+            const float *ot = ota + ((size_t)o * n + s) * ns;
+            float vt = 0.0f;
+            bool end = false;
+            for (unsigned l0 = 0; l0 < ns && !end; l0 += 4) {
+                int sp[4];
+                float w[4], g[4];
+#pragma unroll
+                for (unsigned e = 0; e < 4; e++) {
+                    const unsigned l = min(l0 + e, ns - 1);
+                    sp[e] = rw[l];
+                    w[e] = ot[l];
                 }
-                al = __fadd_rn(al, __fmul_rn(vt, gamma));
+#pragma unroll
+                for (unsigned e = 0; e < 4; e++)
+                    g[e] = Gj[max(sp[e], 0)];
+#pragma unroll
+                for (unsigned e = 0; e < 4; e++) {
+                    end = end || l0 + e >= ns || sp[e] < 0;
+                    vt = end ? vt : __fadd_rn(vt, __fmul_rn(w[e], g[e]));
+                }
+            }
+            return __fmul_rn(vt, gamma);
+        };
+        const bool split = z * n <= (unsigned)kFS;
+        if (split) {
+            for (unsigned x = t; x < z * n; x += kPB)
+                sc[x] = inner(x / n, x % n);
+            __syncthreads();
+        }
+        for (unsigned s = t; s < n; s += kPB) {
+            float al = Rall[(size_t)s * m + a];
+            if (split) {
+#pragma unroll 8
+                for (unsigned o = 0; o < z; o++)
+                    al = __fadd_rn(al, sc[o * n + s]);
+            } else {
+                for (unsigned o = 0; o < z; o++)
+                    al = __fadd_rn(al, inner(o, s));
             }
             alpha[s] = al;
         }
         __syncthreads();
-        if (t == 0) {
+        if (t < 64) {
+            // the products of 64 support entries at a time, then their sum in order
             float v = 0.0f;
-            for (int k = 0; k < kEnd; k++)
-                v = __fadd_rn(v, __fmul_rn(alpha[L.sK[k]], L.bK[k]));
-            P.aval[(size_t)i * m + a] = v;
-            actVal = v;
+            for (int k0 = 0; k0 < kEnd; k0 += 64) {
+                const int k = min(k0 + (int)t, kEnd - 1);
+                const float p = __fmul_rn(alpha[L.sK[k]], L.bK[k]);
+                const int cnt = min(64, kEnd - k0);
+                for (int e = 0; e < cnt; e++)
+                    v = __fadd_rn(v, __int_as_float(
+                        __builtin_amdgcn_readlane(__float_as_int(p), e)));
+            }
+            if (t == 0) {
+                P.aval[(size_t)i * m + a] = v;
+                actVal = v;
+            }
         }
         __syncthreads();
         const float v = actVal;
