@@ -81,7 +81,8 @@ struct PbviInst {
     int *act;
     int *recJ;             // optional per-iteration record: recJ[(iter*r + i)*z + o] = j*
     int *recA;             // and recA[iter*r + i] = chosen action (-1: none)
-    int fused;             // each iteration is one pbvi_fused launch (small instances)
+    int fused;             // action groups of the one pbvi_fused launch that each iteration of a
+                           // small instance is, or 0
     int actionMajor;       // matrix-core scorers: workgroups enumerate (action, belief) with the
                            // action slower, so that concurrent ones read one action's O rows
 };
@@ -250,12 +251,14 @@ struct SupportLds {
     int otU[kUMax];           // s_k*ns + l of pair u (offset into an OT plane)
 };
 
-// Fills the SupportLds of belief i and action a cooperatively (all kPB lanes).
-__device__ void build_support(SupportLds &L, unsigned i, unsigned a, unsigned m, unsigned ns,
-        unsigned rz, const int *__restrict__ S, const int *__restrict__ Z,
-        const float *__restrict__ B, int *cnt)
+// Fills the support (SupportLds or FusedSupport) of belief i and action a cooperatively: lanes
+// t = 0..kPB-1. Its barriers depend on the belief alone, so groups of kPB lanes of one workgroup
+// may fill supports of one belief's actions side by side.
+template <typename SL>
+__device__ __forceinline__ void build_support(SL &L, unsigned i, unsigned a, unsigned m,
+        unsigned ns, unsigned rz, const int *__restrict__ S, const int *__restrict__ Z,
+        const float *__restrict__ B, int *cnt, unsigned t)
 {
-    const unsigned t = threadIdx.x;
     if (t == 0)
         L.kEnd = (int)rz;
     __syncthreads();
@@ -437,7 +440,7 @@ __global__ __launch_bounds__(kPB) void pbvi_score(const PbviInst *__restrict__ i
         kEnd = 0;
         uEnd = 0;
     } else if (EXACT) {
-        build_support(L, i, a, m, ns, P.rz, P.S, P.Z, P.B, scratch);
+        build_support(L, i, a, m, ns, P.rz, P.S, P.Z, P.B, scratch, t);
         kEnd = L.kEnd;
         uEnd = L.uEnd;
     } else {
@@ -1724,36 +1727,63 @@ constexpr int kFN = 2048;          // max states: the alpha and the best alpha i
 constexpr int kFZ = 256;           // max observations
 constexpr int kFS = 6144;          // max observations x alphas: the scores in LDS
 constexpr int kFStage = 24576;     // max words of Gamma, O*T, S, R and the belief in LDS
+constexpr int kFGroups = 4;        // most action groups of kPB lanes in a workgroup
+constexpr size_t kFLds = 160 * 1024;
 
 // dst[x] = get(x) for x < count, eight values per lane requested before any is stored
 template <typename T, typename F>
-__device__ __forceinline__ void fused_stage_copy(T *dst, F get, unsigned count, unsigned t)
+__device__ __forceinline__ void fused_stage_copy(T *dst, F get, unsigned count, unsigned t,
+                                                 unsigned lanes)
 {
-    for (unsigned x0 = t; x0 < count; x0 += 8 * kPB) {
+    for (unsigned x0 = t; x0 < count; x0 += 8 * lanes) {
         T v[8];
 #pragma unroll
         for (int u = 0; u < 8; u++)
-            v[u] = get(min(x0 + u * kPB, count - 1));
+            v[u] = get(min(x0 + u * lanes, count - 1));
 #pragma unroll
         for (int u = 0; u < 8; u++)
-            if (x0 + u * kPB < count)
-                dst[x0 + u * kPB] = v[u];
+            if (x0 + u * lanes < count)
+                dst[x0 + u * lanes] = v[u];
     }
+}
+
+// One action group's part of the dynamic LDS (fused_group_words): its support, the scores (or
+// the inner sums of the alpha), the alpha and the chosen alphas.
+struct FusedSupport {
+    int &kEnd, &uEnd;
+    int *sK;
+    float *bK;
+    int *startK, *spU, *otU;
+};
+
+// Words of a group: 4 (kEnd, uEnd, its value, pad), sK, bK, startK, counts, the pairs, scores,
+// alpha and j*
+__host__ __device__ inline unsigned fused_score_words(unsigned n, unsigned z, unsigned r)
+{
+    const unsigned inner = z * n <= (unsigned)kFS ? z * n : 0u;
+    return max(z * r, inner);
+}
+__host__ __device__ inline unsigned fused_group_words(unsigned n, unsigned ns, unsigned z,
+                                                      unsigned r, unsigned rz)
+{
+    return 4 + 4 * rz + 2 + 2 * rz * ns + fused_score_words(n, z, r) + n + z;
 }
 
 // The scores of every (observation, alpha): lane t takes alpha t mod jl (jl a power of two) and Q
 // observations at a time, kPB / jl apart, so one read of Gamma serves Q sums. The support's
 // pairs are the same for every lane; four of them are read together, then their Gamma and O*T
 // values, then their sums follow in the reference's order. At one wave per SIMD the chains of
-// LDS reads were the iteration's time.
+// LDS reads were the iteration's time: with them and the actions one after another, nova's CPU
+// case (n = 64, m = 4, z = 8, ns = 4, r = 128, rz = 8) took 84.5 us an iteration; with batched
+// reads (here and for the alpha's inner sums) 39.9 us, with four actions side by side 19.0 us.
 template <int Q>
-__device__ __forceinline__ void fused_scores(const SupportLds &L, const float *ota,
+__device__ __forceinline__ void fused_scores(const FusedSupport &L, const float *ota,
         const float *G, float *sc, unsigned n, unsigned ns, unsigned z, unsigned r, unsigned gs,
-        unsigned jl, float gamma)
+        unsigned jl, float gamma, unsigned t)
 {
-    const unsigned groups = kPB / jl, og = threadIdx.x / jl, plane = n * ns;
+    const unsigned groups = kPB / jl, og = t / jl, plane = n * ns;
     const int kEnd = __builtin_amdgcn_readfirstlane(L.kEnd);
-    for (unsigned j0 = threadIdx.x % jl; j0 < r; j0 += jl) {
+    for (unsigned j0 = t % jl; j0 < r; j0 += jl) {
         const float *Gj = G + (size_t)j0 * gs;
         for (unsigned o0 = og; o0 < z; o0 += Q * groups) {
             const float *ot[Q];
@@ -1807,16 +1837,10 @@ __device__ __forceinline__ void fused_scores(const SupportLds &L, const float *o
     }
 }
 
-__global__ __launch_bounds__(kPB) void pbvi_fused(const PbviInst *__restrict__ insts,
+__global__ __launch_bounds__(kFGroups * kPB) void pbvi_fused(const PbviInst *__restrict__ insts,
         const unsigned *__restrict__ off, unsigned count, unsigned iter, unsigned flip)
 {
-    __shared__ SupportLds L;
-    __shared__ int scratch[kKMax + 1];
-    __shared__ float sc[kFS];
-    __shared__ float alpha[kFN], bestAlpha[kFN];
-    __shared__ int js[kFZ], bestJs[kFZ];
-    __shared__ float actVal;
-    extern __shared__ float stage[];   // Gamma, O*T, S, R and belief i: fused_stage_words
+    extern __shared__ float stage[];   // fused_stage_words, then fused_group_words per group
     if (blockIdx.x >= off[count])
         return;   // a grid larger than the plan's workgroups does nothing
     const unsigned b = find_inst(off, count, blockIdx.x);
@@ -1825,7 +1849,9 @@ __global__ __launch_bounds__(kPB) void pbvi_fused(const PbviInst *__restrict__ i
         return;
     const unsigned n = P.n, ns = P.ns, m = P.m, z = P.z, r = P.r;
     const float gamma = P.gamma;
-    const unsigned i = blockIdx.x - off[b], t = threadIdx.x;
+    const unsigned i = blockIdx.x - off[b];
+    const unsigned all = threadIdx.x, lanes = blockDim.x;
+    const unsigned t = all % kPB, group = all / kPB;      // P.fused groups take an action each
     // one round of loads stages everything the iteration reads: Gamma [r][n], O*T [m][z][n][ns],
     // S [m][n][ns] (action-major), R [n][m] and belief i's (Z, B)
     const unsigned rz = P.rz, zn = z * n * ns, sn = n * ns;
@@ -1842,49 +1868,66 @@ __global__ __launch_bounds__(kPB) void pbvi_fused(const PbviInst *__restrict__ i
         // eight loads per lane requested before any is stored (one instance's staging is the
         // kernel's latency at these sizes)
         const float *__restrict__ Gsrc = src_gamma(P, iter, flip);
-        for (unsigned x0 = t; x0 < r * n; x0 += 8 * kPB) {
+        for (unsigned x0 = all; x0 < r * n; x0 += 8 * lanes) {
             float v[8];
 #pragma unroll
             for (int u = 0; u < 8; u++)
-                v[u] = Gsrc[min(x0 + u * kPB, r * n - 1)];
+                v[u] = Gsrc[min(x0 + u * lanes, r * n - 1)];
 #pragma unroll
             for (int u = 0; u < 8; u++) {
-                const unsigned x = x0 + u * kPB;
+                const unsigned x = x0 + u * lanes;
                 if (x < r * n)
                     G[(x / n) * gs + x % n] = v[u];
             }
         }
-        fused_stage_copy(OTall, [&](unsigned x) { return P.OT[x]; }, m * zn, t);
+        fused_stage_copy(OTall, [&](unsigned x) { return P.OT[x]; }, m * zn, all, lanes);
         fused_stage_copy(Sall, [&](unsigned x) {
             const unsigned a = x / sn, e = x % sn;
             return P.S[((size_t)(e / ns) * m + a) * ns + e % ns];
-        }, m * sn, t);
-        fused_stage_copy(Rall, [&](unsigned x) { return P.R[x]; }, n * m, t);
-        for (unsigned k = t; k < rz; k += kPB) {
+        }, m * sn, all, lanes);
+        fused_stage_copy(Rall, [&](unsigned x) { return P.R[x]; }, n * m, all, lanes);
+        for (unsigned k = all; k < rz; k += lanes) {
             Zi[k] = P.Z[(size_t)i * rz + k];
             Bi[k] = P.B[(size_t)i * rz + k];
         }
     }
+    const unsigned groups = (unsigned)P.fused;
+    const unsigned words = fused_group_words(n, ns, z, r, rz);
+    float *bestAlpha = Bi + rz;
+    int *bestJs = reinterpret_cast<int *>(bestAlpha + n);
+    float *groupBase = reinterpret_cast<float *>(bestJs + z);
+    float *mine = groupBase + (size_t)min(group, groups - 1) * words;
+    int *mi = reinterpret_cast<int *>(mine);
+    FusedSupport L{mi[0], mi[1], mi + 4, mine + 4 + rz, mi + 4 + 2 * rz, mi + 4 + 4 * rz + 2,
+                   mi + 4 + 4 * rz + 2 + rz * ns};
+    int *scratch = mi + 4 + 3 * rz + 1;
+    float *sc = mine + 4 + 4 * rz + 2 + 2 * rz * ns;
+    float *alpha = sc + fused_score_words(n, z, r);
+    int *js = reinterpret_cast<int *>(alpha + n);
     float bestValue = kLow;            // the same in every lane
     int bestA = -1;
-    for (unsigned a = 0; a < m; a++) {
+    for (unsigned a0 = 0; a0 < m; a0 += groups) {
+        // the round's actions side by side; a group without one repeats the last action (its
+        // lanes keep the barriers whole, its writes repeat that action's) and is left out of the
+        // choice below
+        const unsigned a = min(a0 + group, m - 1);
         const float *ota = OTall + (size_t)a * zn;
         const int *Sa = Sall + (size_t)a * sn;
         // the support's pairs from the staged rows (belief 0 of one action: i = 0, m = 1,
         // a = 0); build_support reads its inputs only after its first barrier, which orders
         // the staging above before them
-        build_support(L, 0, 0, 1, ns, rz, Sa, Zi, Bi, scratch);   // ends with a barrier
+        build_support(L, 0, 0, 1, ns, rz, Sa, Zi, Bi, scratch, t);   // ends with a barrier
         const int kEnd = L.kEnd;
         // score of alpha j under observation o: sum_k ((sum_l (O*T) * Gamma[j, sp]) * gamma) * b_k
         {
             const unsigned jl = min((unsigned)kPB, 1u << (32 - __clz((int)max(r, 2u) - 1)));
-            const unsigned groups = kPB / jl;
-            if (z <= groups)
-                fused_scores<1>(L, ota, G, sc, n, ns, z, r, gs, jl, gamma);
-            else if (z <= 2 * groups)
-                fused_scores<2>(L, ota, G, sc, n, ns, z, r, gs, jl, gamma);
+            const unsigned across = kPB / jl;
+            if (z <= across)
+                fused_scores<1>(L, ota, G, sc, n, ns, z, r, gs, jl, gamma, t);
+            else if (z <= 2 * across)
+                fused_scores<2>(L, ota, G, sc, n, ns, z, r, gs, jl, gamma, t);
             else
-                fused_scores<4>(L, ota, G, sc, n, ns, z, r, gs, jl, gamma);
+                fused_scores<4>(L, ota, G, sc, n, ns, z, r, gs, jl, gamma, t);
         }
         __syncthreads();
         // first maximiser per observation by strict '>' from -1e10 (none: alpha 0): 32 lanes
@@ -1976,22 +2019,29 @@ __global__ __launch_bounds__(kPB) void pbvi_fused(const PbviInst *__restrict__ i
             }
             if (t == 0) {
                 P.aval[(size_t)i * m + a] = v;
-                actVal = v;
+                mine[2] = v;
             }
         }
         __syncthreads();
-        const float v = actVal;
-        if (v > bestValue) {
-            bestValue = v;
-            bestA = (int)a;
-            for (unsigned s = t; s < n; s += kPB)
-                bestAlpha[s] = alpha[s];
-            for (unsigned o = t; o < z; o += kPB)
-                bestJs[o] = js[o];
+        int bestG = -1;                // the round's winner by strict '>', lower actions first
+        for (unsigned g = 0; g < groups && a0 + g < m; g++) {
+            const float v = groupBase[(size_t)g * words + 2];
+            if (v > bestValue) {
+                bestValue = v;
+                bestA = (int)(a0 + g);
+                bestG = (int)g;
+            }
+        }
+        if (bestG >= 0) {
+            const float *from = groupBase + (size_t)bestG * words + (alpha - mine);
+            for (unsigned s = all; s < n; s += lanes)
+                bestAlpha[s] = from[s];
+            for (unsigned o = all; o < z; o += lanes)
+                bestJs[o] = reinterpret_cast<const int *>(from + n)[o];
         }
         __syncthreads();
     }
-    if (t == 0) {
+    if (all == 0) {
         P.act[i] = bestA;
         if (bestA >= 0)
             P.pi[i] = (unsigned)bestA;
@@ -1999,12 +2049,12 @@ __global__ __launch_bounds__(kPB) void pbvi_fused(const PbviInst *__restrict__ i
             P.recA[(size_t)iter * r + i] = bestA;
     }
     if (P.recJ != nullptr)
-        for (unsigned o = t; o < z; o += kPB)
+        for (unsigned o = all; o < z; o += lanes)
             P.recJ[((size_t)iter * r + i) * z + o] = (bestA >= 0) ? bestJs[o] : -1;
     if (bestA >= 0) {
         // no action beat -1e10: Gamma'[i] and pi[i] keep their values
         float *out = dst_gamma(P, iter, flip) + (size_t)i * n;
-        for (unsigned s = t; s < n; s += kPB)
+        for (unsigned s = all; s < n; s += lanes)
             out[s] = bestAlpha[s];
     }
 }
@@ -2294,29 +2344,43 @@ static double fused_stage_words(const PbviInst &I)
            (double)I.n * I.m + 2.0 * I.rz;
 }
 
-// Whether a PBVI instance runs its iterations as single pbvi_fused launches: sparse modes, the
-// kernel's LDS bounds and the exact mode's support staging, and at most 256 (fast mode) or
-// 1024 (exact mode) scoring multiply-adds per lane and iteration, m * ceil(z*r / 256) * rz*ns.
-// Measured on nova's domains, the one launch takes 14-21 us per iteration at tiger, paint and
-// shuttle (24-28 us with four kernels, fast mode) and 61 us at 4x3 (35 us fast, 83 us exact);
-// at aloha and tiger_grid it is 3-5x slower than fast mode's four kernels.
+// Dynamic LDS of pbvi_fused with `groups` action groups (with one group always within kFLds).
+static size_t fused_lds(const PbviInst &I, int groups)
+{
+    return sizeof(float) * ((size_t)fused_stage_words(I) + I.n + I.z +
+                            (size_t)groups * fused_group_words(I.n, I.ns, I.z, I.r, I.rz));
+}
+
+// The action groups of a PBVI instance's pbvi_fused launches (as many as its actions and the LDS
+// allow), or 0 when it does not run its iterations as such. It does in the sparse modes, within
+// the kernel's LDS bounds and the exact mode's support staging, and with at most 256 (fast mode)
+// or 1,536 (exact mode) scoring multiply-adds per lane of one group and iteration,
+// m * ceil(z*r / 256) * rz*ns. us per iteration, one launch / four kernels, by that number:
+// exact 432: 32 / 56, 1,170: 46 / 66, 1,512: 48 / 79, 1,824: 81 / 65; fast 224: 15 / 24,
+// 252: 18 / 24, 264: 26 / 24, 672: 57 / 27.
 // NOVA_AMD_PBVI_FUSED=0 turns it off; another value replaces the limit of both modes.
-static bool fused_fits(const PbviInst &I, int mode)
+static int fused_fits(const PbviInst &I, int mode)
 {
     if (mode != 0 && mode != 1)
-        return false;
-    double limit = (mode == 1) ? 1024.0 : 256.0;
+        return 0;
+    double limit = (mode == 1) ? 1536.0 : 256.0;
     if (const char *f = std::getenv("NOVA_AMD_PBVI_FUSED"))
         limit = std::atof(f);
     if (limit <= 0.0)
-        return false;
+        return 0;
     const size_t zr = (size_t)I.z * I.r;
     const double perLane = (double)I.m * (double)((zr + kPB - 1) / kPB) * I.rz * I.ns;
     const double stage = fused_stage_words(I);
-    return I.rb == I.r && I.n <= (unsigned)kFN && I.z <= (unsigned)kFZ &&
+    const bool fits = I.rb == I.r && I.n <= (unsigned)kFN && I.z <= (unsigned)kFZ &&
            (size_t)I.z * I.r <= (size_t)kFS && I.rz <= (unsigned)kKMax &&
            (size_t)I.rz * I.ns <= (size_t)kUMax && stage <= (double)kFStage &&
            perLane <= limit;
+    if (!fits)
+        return 0;
+    int groups = 1;
+    while (2 * groups <= kFGroups && 2u * groups <= I.m && fused_lds(I, 2 * groups) <= kFLds)
+        groups *= 2;
+    return groups;
 }
 
 // A launch plan over a set of instances: device descriptors and per-stage offsets.
@@ -2333,6 +2397,7 @@ struct PbviPlan {
     unsigned *dOff = nullptr;        // [tr | sc(jpt=1) | ... | sc(32) | be | fu], count+1 each
     unsigned totTr = 0, totSc[kVariants] = {}, totBe = 0, totFu = 0;
     size_t fuLds = 0;                // dynamic LDS of pbvi_fused: the largest fused instance's
+    int fuGroups = 0;                // its action groups, the same for every fused instance
     size_t ldsBytes = 0;
     size_t actLds = 2 * sizeof(float) * kKMax;   // dynamic LDS of pbvi_action
     unsigned maxHorizon = 0;
@@ -2394,8 +2459,15 @@ static int plan_upload(PbviPlan &pl, void *dst, hipStream_t st, const char *fn)
         scs[v] = &off[(1 + v) * (c + 1)];
     pl.ldsBytes = 0;
     pl.maxHorizon = 0;
+    // one launch has one width: every fused instance runs with the fewest groups among them
+    pl.fuGroups = 0;
+    for (const PbviInst &I : pl.host)
+        if (I.fused)
+            pl.fuGroups = pl.fuGroups ? std::min(pl.fuGroups, I.fused) : I.fused;
     for (unsigned b = 0; b < c; b++) {
         PbviInst &I = pl.host[b];
+        if (I.fused)
+            I.fused = pl.fuGroups;
         I.tiles = tiles_for(I.r, I.jpt);
         const bool four = !I.fused;
         tr[b + 1] = tr[b] + (four ? ((I.n + 63) / 64) * (I.rS / 64) : 0u);
@@ -2408,7 +2480,7 @@ static int plan_upload(PbviPlan &pl, void *dst, hipStream_t st, const char *fn)
         be[b + 1] = be[b] + (four ? I.rb : 0u);
         fu[b + 1] = fu[b] + (four ? 0u : I.rb);
         if (!four)
-            pl.fuLds = std::max(pl.fuLds, sizeof(float) * (size_t)fused_stage_words(I));
+            pl.fuLds = std::max(pl.fuLds, fused_lds(I, pl.fuGroups));
         if (I.useLds && four)
             pl.ldsBytes = std::max(pl.ldsBytes, sizeof(float) * (size_t)I.n);
         if (four)
@@ -2429,7 +2501,7 @@ static int plan_upload(PbviPlan &pl, void *dst, hipStream_t st, const char *fn)
                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl.actLds);
     if (ea == hipSuccess && pl.totFu > 0)
         ea = hipFuncSetAttribute((const void *)pbvi_fused,
-                                 hipFuncAttributeMaxDynamicSharedMemorySize, 4 * kFStage);
+                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)kFLds);
     if (ea != hipSuccess)
         return hip_fail(ea, fn, "Failed to set up the one-launch PBVI kernel.",
                         NOVA_ERROR_KERNEL_EXECUTION);
@@ -2558,7 +2630,7 @@ static void plan_enqueue(const PbviPlan &pl, unsigned iter, unsigned flip, int m
     const unsigned *tr = pl.dOff, *be = pl.dOff + (kVariants + 1) * (c + 1);
     const unsigned *fu = pl.dOff + (kVariants + 2) * (c + 1);
     if (pl.totFu > 0)
-        hipLaunchKernelGGL(pbvi_fused, dim3(pl.totFu), dim3(kPB), pl.fuLds, st, pl.dInst, fu, c,
+        hipLaunchKernelGGL(pbvi_fused, dim3(pl.totFu), dim3(kPB * pl.fuGroups), pl.fuLds, st, pl.dInst, fu, c,
                            iter, flip);
     if (pl.totBe == 0)
         return;
@@ -3013,7 +3085,7 @@ static int pbvi_run_iters(const nova::POMDP *p, nova::POMDPPBVIGPU *pb, unsigned
     fill_inst(p, pl.host[0], pb->d_Gamma, pb->d_GammaPrime, pb->d_pi,
               reinterpret_cast<char *>(pb->d_alphaBA), kNoHorizon);
     pl.host[0].jpt = jpt;
-    pl.host[0].fused = (dense == nullptr && fused_fits(pl.host[0], mode)) ? 1 : 0;
+    pl.host[0].fused = dense == nullptr ? fused_fits(pl.host[0], mode) : 0;
     const bool hit = g_pgraph.exec && g_pgraph.iters == iters && g_pgraph.flip == flip &&
                      g_pgraph.gamma == p->gamma && g_pgraph.mode == mode &&
                      g_pgraph.jpt == jpt && g_pgraph.fused == pl.host[0].fused &&
@@ -3336,8 +3408,8 @@ int pomdp_pbvi_profile_gpu(const POMDP *pomdp, POMDPPBVIGPU *pbvi, float *stageM
     fill_inst(pomdp, pl.host[0], pbvi->d_Gamma, pbvi->d_GammaPrime, pbvi->d_pi,
               reinterpret_cast<char *>(pbvi->d_alphaBA), kNoHorizon);
     pl.host[0].jpt = S->jpt;
-    pl.host[0].fused = (dense_for(pbvi->d_alphaBA) == nullptr &&
-                        fused_fits(pl.host[0], S->mode)) ? 1 : 0;
+    pl.host[0].fused = dense_for(pbvi->d_alphaBA) == nullptr
+                           ? fused_fits(pl.host[0], S->mode) : 0;
     rc = plan_upload(pl, plain_plan_mem(pomdp, pbvi), st, fn);
     if (rc != NOVA_SUCCESS)
         return rc;
@@ -3376,7 +3448,7 @@ int pomdp_pbvi_profile_gpu(const POMDP *pomdp, POMDPPBVIGPU *pbvi, float *stageM
         // a small instance: the whole iteration is one launch, reported as the score stage
         hipEventRecord(ev[0], st);
         hipEventRecord(ev[1], st);
-        hipLaunchKernelGGL(pbvi_fused, dim3(pl.totFu), dim3(kPB), pl.fuLds, st, pl.dInst,
+        hipLaunchKernelGGL(pbvi_fused, dim3(pl.totFu), dim3(kPB * pl.fuGroups), pl.fuLds, st, pl.dInst,
                            pl.dOff + (kVariants + 2) * (c + 1), c, 0u, flip);
         hipEventRecord(ev[2], st);
         hipEventRecord(ev[3], st);
@@ -3444,7 +3516,7 @@ int pomdp_pbvi_run_recorded_gpu(const POMDP *pomdp, POMDPPBVIGPU *pbvi, unsigned
     pl.host[0].jpt = S->jpt;
     pl.host[0].recJ = d_recJ;
     pl.host[0].recA = d_recA;
-    pl.host[0].fused = fused_fits(pl.host[0], S->mode) ? 1 : 0;
+    pl.host[0].fused = fused_fits(pl.host[0], S->mode);
     rc = plan_upload(pl, plain_plan_mem(pomdp, pbvi), st, fn);
     if (rc != NOVA_SUCCESS)
         return rc;
@@ -3499,7 +3571,7 @@ int pomdp_pbvi_batch_execute_gpu(const POMDP *const *pomdps, POMDPPBVIGPU *const
                       pbvis[b]->d_pi, reinterpret_cast<char *>(pbvis[b]->d_alphaBA),
                       pomdps[b]->horizon);
             pl.host[b].jpt = plain_jpt(pbvis[b]->d_alphaBA);
-            pl.host[b].fused = fused_fits(pl.host[b], g_pbvi_mode) ? 1 : 0;
+            pl.host[b].fused = fused_fits(pl.host[b], g_pbvi_mode);
         }
         rc = plan_upload(pl, planMem, st, fn);
     }

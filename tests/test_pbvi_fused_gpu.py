@@ -110,6 +110,22 @@ def test_exact_fused_equals_four_kernels_and_oracle(oracle, monkeypatch, name):
           % (name, steps), flush=True)
 
 
+@pytest.mark.parametrize("n,m,z,ns,r,rz", [
+    (40, 2, 3, 3, 20, 5), (30, 3, 17, 4, 15, 30), (33, 5, 4, 5, 300, 12), (90, 7, 2, 2, 9, 80),
+    (64, 4, 1, 8, 256, 1), (20, 8, 40, 3, 33, 7),
+])
+def test_action_groups_equal_four_kernels(monkeypatch, n, m, z, ns, r, rz):
+    """Two or four actions of a belief side by side: rounds that are not full, supports above and
+    below a wave, entries of more than four pairs, observations in one to several sweeps."""
+    P = ragged(synth.pomdp_arrays(n=n, m=m, z=z, ns=ns, r=r, rz=rz, seed=n + m, horizon=1,
+                                  gamma=0.95), n)
+    fused = updates(P, EXACT, 4)
+    monkeypatch.setenv("NOVA_AMD_PBVI_FUSED", "0")
+    for t, (a, b) in enumerate(zip(fused, updates(P, EXACT, 4))):
+        assert np.array_equal(bits(a[0]), bits(b[0])), t
+        assert all(np.array_equal(x, y) for x, y in zip(a[1:], b[1:])), t
+
+
 @pytest.mark.parametrize("name", ["tiny", "mid", "n_above_block"])
 def test_fast_fused_equals_float_oracle(oracle, name):
     P = instance(name)
