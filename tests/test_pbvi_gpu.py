@@ -298,6 +298,22 @@ def test_exact_batched_paths_bitwise_vs_oracle(oracle, ns):
     assert np.array_equal(bits(G), bits(Go)) and np.array_equal(pi, pio)
 
 
+@pytest.mark.parametrize("n,ns", [(1, 1), (1023, 2), (1025, 5), (2048, 8), (2049, 4), (4096, 3),
+                                  (4097, 8), (5120, 7), (5121, 8), (8192, 4), (8193, 4),
+                                  (9000, 8), (600, 9)])
+def test_exact_materialization_sizes_bitwise_vs_oracle(oracle, monkeypatch, n, ns):
+    """Exact runs at the edges of the materialization's lanes (1 to 8 states a lane, up to four or
+    eight successors; the larger models and longer lists keep the general loop), with ragged
+    lists: Gamma and pi equal the oracle's bit for bit."""
+    monkeypatch.setenv("NOVA_AMD_PBVI_FUSED", "0")
+    ns = min(ns, n)
+    P = ragged(synth.pomdp_arrays(n=n, m=2, z=3, ns=ns, r=9, rz=min(6, n), seed=n + ns,
+                                  gamma=0.95, horizon=2), n, frac=0.3)
+    G, pi = gpu_solve(P, EXACT, horizon=2)
+    Go, pio = oracle.pbvi_run(P, horizon=2)
+    assert np.array_equal(bits(G), bits(Go)) and np.array_equal(pi, pio)
+
+
 @pytest.mark.parametrize("n,m,z,ns,r,rz,horizon,seed", [
     (200, 3, 5, 20, 40, 40, 4, 61),      # 800 pairs per (belief, action): two support chunks
     (900, 2, 4, 3, 20, 700, 3, 62),      # rz > 512 entries, ns = 3
