@@ -89,25 +89,62 @@ __global__ __launch_bounds__(kB) void mu_init(unsigned n, unsigned rz, const int
     }
 }
 
-// u[i][s'] = sum over predecessors (s, l) of s' under a_i of T(s,a_i,l) mu[i][s]
-__global__ __launch_bounds__(kB) void pred_gather(unsigned n, unsigned r,
+// u[i][s'] = sum over predecessors (s, l) of s' under a_i of T(s,a_i,l) mu[i][s], one workgroup per
+// alpha with mu[i] in LDS where it fits (useLds), a lane's list entries requested kPredBatch at
+// a time. One entry at a time with mu gathered from L2, each lane was a chain of two loads per
+// entry: 220 us for r = 1,024, n = 5,000, ns = 8, now 107 us.
+constexpr unsigned kPredThreads = 1024;
+constexpr unsigned kPredBatch = 8;
+constexpr unsigned kPredLds = 36 * 1024;         // states of mu in LDS (144 KB)
+
+__global__ __launch_bounds__(kPredThreads) void pred_gather(unsigned n,
         const int *__restrict__ act, const unsigned *__restrict__ pstart,
         const int *__restrict__ pS, const float *__restrict__ pT, const float *__restrict__ mu,
-        float *__restrict__ u)
+        float *__restrict__ u, int useLds)
 {
-    const unsigned i = blockIdx.y;
-    const unsigned sp = blockIdx.x * kB + threadIdx.x;
-    if (sp >= n)
-        return;
+    extern __shared__ float row[];
+    const unsigned i = blockIdx.x, t = threadIdx.x;
     const int a = act[i];
-    float acc = 0.0f;
-    if (a >= 0) {
-        const unsigned *ps = pstart + (size_t)a * (n + 1);
-        const float *mi = mu + (size_t)i * n;
-        for (unsigned q = ps[sp]; q < ps[sp + 1]; q++)
-            acc += pT[q] * mi[pS[q]];
+    const float *mi = mu + (size_t)i * n;
+    float *ui = u + (size_t)i * n;
+    if (a < 0) {
+        for (unsigned sp = t; sp < n; sp += kPredThreads)
+            ui[sp] = 0.0f;
+        return;
     }
-    u[(size_t)i * n + sp] = acc;
+    if (useLds) {
+        for (unsigned s = t; s < n; s += kPredThreads)
+            row[s] = mi[s];
+        __syncthreads();
+    }
+    const unsigned *ps = pstart + (size_t)a * (n + 1);
+    for (unsigned sp = t; sp < n; sp += kPredThreads) {
+        const unsigned lo = ps[sp], hi = ps[sp + 1];
+        float acc = 0.0f;
+        for (unsigned q0 = lo; q0 < hi; q0 += kPredBatch) {
+            int si[kPredBatch];
+            float tv[kPredBatch];
+#pragma unroll
+            for (unsigned e = 0; e < kPredBatch; e++) {
+                const unsigned q = min(q0 + e, hi - 1);
+                si[e] = pS[q];
+                tv[e] = pT[q];
+            }
+            if (useLds) {
+#pragma unroll
+                for (unsigned e = 0; e < kPredBatch; e++)
+                    tv[e] = tv[e] * row[si[e]];
+            } else {
+#pragma unroll
+                for (unsigned e = 0; e < kPredBatch; e++)
+                    tv[e] = tv[e] * mi[si[e]];
+            }
+#pragma unroll
+            for (unsigned e = 0; e < kPredBatch; e++)
+                acc = q0 + e < hi ? acc + tv[e] : acc;
+        }
+        ui[sp] = acc;
+    }
 }
 
 // dR[s][a] += sum over alphas i with a_i = a of mu[i][s]  (lists per action)
@@ -396,11 +433,16 @@ int pomdp_pbvi_replay_grad_gpu(const POMDP *pomdp, unsigned int iterations, cons
         hipLaunchKernelGGL(mu_init, dim3(r), dim3(kB), 0, st, n, pomdp->rz, pomdp->d_Z,
                            pomdp->d_B, dfs, dfl, muA);
         const dim3 g((n + kB - 1) / kB, r), ga((n + kB - 1) / kB, m);
+        const int predLds = n <= kPredLds ? 1 : 0;
+        hipFuncSetAttribute((const void *)pred_gather,
+                            hipFuncAttributeMaxDynamicSharedMemorySize, 4 * kPredLds);
         for (int t = (int)H - 1; t >= 0; t--) {
             const int *act = d_recA + (size_t)t * r;
             hipLaunchKernelGGL(dr_accumulate, ga, dim3(kB), 0, st, n, m,
                                das + (size_t)t * (m + 1), dal, muA, d_dR);
-            hipLaunchKernelGGL(pred_gather, g, dim3(kB), 0, st, n, r, act, dps, dpS, dpT, muA, u);
+            hipLaunchKernelGGL(pred_gather, dim3(r), dim3(kPredThreads),
+                               predLds ? sizeof(float) * n : 0, st, n, act, dps, dpS, dpT, muA, u,
+                               predLds);
             const unsigned *ssT = &sstart[(size_t)t * (r + 1)];
             const unsigned segBase = ssT[0], segs = ssT[r] - ssT[0];
             // in slices of at most 65,535 segments (the grid's y extent)
