@@ -32,11 +32,12 @@ extern "C" int mdp_vi_sweep_kernel_gpu(const MDP *mdp, const MDPVIGPU *vi, unsig
 // Batched value iteration (no counterpart in the reference): solves count MDPs (each resident
 // on the device, each with its own horizon, gamma and solver struct, VInitial or zeros) exactly
 // as mdp_vi_execute_gpu would solve each one (mdp_vi_cpu.cpp:36-63 per sweep; V and pi bit for
-// bit), with every sweep of every instance captured into one HIP graph: one launch per sweep
-// for all instances, over a grid of every instance's state tiles. m <= 1024 per instance.
+// bit), with one launch per sweep for all instances, over a grid of every instance's state
+// tiles, and their values and policies moved in one piece. m <= 1024 per instance. Solver
+// structs whose device buffers already have their model's size keep them.
 // policies (nullable) is an array of count empty policy structs that receive the results;
 // the solver structs keep V/V'/pi on the device as after an initialize and the sweeps
-// (currentHorizon = horizon). elapsedMs (nullable) gets the device time of the graph.
+// (currentHorizon = horizon). elapsedMs (nullable) gets the device time of the sweeps.
 extern "C" int mdp_vi_batch_execute_gpu(const MDP *const *mdps, MDPVIGPU *const *vis,
         unsigned int count, MDPValueFunction *policies, float *elapsedMs);
 

@@ -809,8 +809,7 @@ __global__ __launch_bounds__(kResThreads) void vi_resident(unsigned n, unsigned 
 
 // ---- batched value iteration: many MDPs of uneven size, one launch per sweep for all
 //
-// Every sweep of every instance is captured into one HIP graph: launch k runs sweep k of all
-// instances whose horizon exceeds k, over one grid holding every instance's tiles (an
+// Launch k runs sweep k of all instances whose horizon exceeds k, over one grid holding every instance's tiles (an
 // instance's workgroups are consecutive; its tile offset comes from a prefix table). A tile
 // is kBatchTile (s, a) rows of whole states, one row per lane, summed in the reference's order,
 // (gamma*T)*V products and sums rounded separately, and one lane per state takes the max over
@@ -921,6 +920,44 @@ __global__ __launch_bounds__(kBatchThreads) void vi_batch_sweep(const ViInst *__
         if (last)
             I.pi[s0 + x] = bestA;
     }
+}
+
+// The batch's initial values and results move in one piece: V0 of all instances lies in `all`,
+// instance b's from base[b] on, and becomes its V and V' (pi = 0); collect takes each
+// instance's last V and pi to the same places of outV and outPi.
+__global__ __launch_bounds__(kBatchThreads) void vi_batch_init(const ViInst *__restrict__ inst,
+        const unsigned *__restrict__ base, unsigned count, const float *__restrict__ all)
+{
+    const unsigned x = blockIdx.x * kBatchThreads + threadIdx.x;
+    if (x >= base[count])
+        return;
+    unsigned lo = 0, hi = count;
+    while (hi - lo > 1) {
+        const unsigned mid = (lo + hi) / 2;
+        if (base[mid] <= x) lo = mid; else hi = mid;
+    }
+    const ViInst &I = inst[lo];
+    const unsigned s = x - base[lo];
+    I.V[s] = I.Vp[s] = all[x];
+    I.pi[s] = 0;
+}
+
+__global__ __launch_bounds__(kBatchThreads) void vi_batch_collect(
+        const ViInst *__restrict__ inst, const unsigned *__restrict__ base, unsigned count,
+        float *__restrict__ outV, unsigned *__restrict__ outPi)
+{
+    const unsigned x = blockIdx.x * kBatchThreads + threadIdx.x;
+    if (x >= base[count])
+        return;
+    unsigned lo = 0, hi = count;
+    while (hi - lo > 1) {
+        const unsigned mid = (lo + hi) / 2;
+        if (base[mid] <= x) lo = mid; else hi = mid;
+    }
+    const ViInst &I = inst[lo];
+    const unsigned s = x - base[lo];
+    outV[x] = (I.horizon % 2 == 0 ? I.V : I.Vp)[s];
+    outPi[x] = I.pi[s];
 }
 
 unsigned pow2_at_least(unsigned x)
@@ -1583,10 +1620,9 @@ static bool mdp_device_ready(const nova::MDP *mdp)
            mdp->d_T != nullptr && mdp->d_R != nullptr;
 }
 
-// mdp_vi_initialize_gpu's work: V, V' (from VInitial or zeros) and pi on the device, and, when
-// layout, the sweep layout the model's size calls for.
-static int vi_state_init(const nova::MDP *mdp, nova::MDPVIGPU *vi, const char *fn,
-                         bool layout)
+// Fresh buffers for V, V' and pi on the device, unfilled (buffers of an earlier initialize are
+// released).
+static int vi_state_alloc(const nova::MDP *mdp, nova::MDPVIGPU *vi, const char *fn)
 {
     if (mdp == nullptr || mdp->n == 0 || vi == nullptr) {
         NOVA_ERR(fn, "Invalid arguments.");
@@ -1608,8 +1644,17 @@ static int vi_state_init(const nova::MDP *mdp, nova::MDPVIGPU *vi, const char *f
         rc = device_alloc((void **)&vi->d_VPrime, n * sizeof(float), fn, "the value function (prime)");
     if (rc == NOVA_SUCCESS)
         rc = device_alloc((void **)&vi->d_pi, n * sizeof(unsigned), fn, "the policy (pi)");
+    return rc;
+}
+
+// mdp_vi_initialize_gpu's work: V, V' (from VInitial or zeros) and pi on the device, and the sweep
+// layout the model's size calls for.
+static int vi_state_init(const nova::MDP *mdp, nova::MDPVIGPU *vi, const char *fn)
+{
+    int rc = vi_state_alloc(mdp, vi, fn);
     if (rc != NOVA_SUCCESS)
         return rc;
+    const size_t n = mdp->n;
 
     std::vector<float> zeros;
     const float *V0 = vi->VInitial;
@@ -1624,7 +1669,7 @@ static int vi_state_init(const nova::MDP *mdp, nova::MDPVIGPU *vi, const char *f
         e = hipMemset(vi->d_pi, 0, n * sizeof(unsigned));
     rc = hip_fail(e, fn, "Failed to copy memory from host to device for V/pi.",
                   NOVA_ERROR_MEMCPY_TO_DEVICE);
-    if (layout && rc == NOVA_SUCCESS && mdp->d_S != nullptr && mdp->d_T != nullptr) {
+    if (rc == NOVA_SUCCESS && mdp->d_S != nullptr && mdp->d_T != nullptr) {
         const int want = layout_wanted(mdp);
         if (want == 2)
             rc = sorted_build(mdp, vi->d_V, stream(), fn);
@@ -1643,7 +1688,7 @@ using namespace nova_amd;
 int mdp_vi_initialize_gpu(const MDP *mdp, MDPVIGPU *vi)
 {
     NOVA_AMD_API_LOCK();
-    return vi_state_init(mdp, vi, "mdp_vi_initialize_gpu", true);
+    return vi_state_init(mdp, vi, "mdp_vi_initialize_gpu");
 }
 
 int mdp_vi_uninitialize_gpu(const MDP *mdp, MDPVIGPU *vi)
@@ -1757,13 +1802,27 @@ int mdp_vi_batch_execute_gpu(const MDP *const *mdps, MDPVIGPU *const *vis, unsig
             return NOVA_ERROR_INVALID_DATA;
         }
     }
-    int rc = NOVA_SUCCESS;
+    int rc = NOVA_SUCCESS, dev = -1;
+    hipGetDevice(&dev);
     std::vector<ViInst> host(count);
-    std::vector<unsigned> off(count + 1, 0);
+    // per instance: first tile, first state in the batch's arrays
+    std::vector<unsigned> off(2 * (size_t)(count + 1), 0);
+    unsigned *base = &off[count + 1];
     unsigned maxH = 0;
     for (unsigned b = 0; b < count && rc == NOVA_SUCCESS; b++) {
         const MDP *mdp = mdps[b];
-        rc = vi_state_init(mdp, vis[b], fn, false);
+        MDPVIGPU *vi = vis[b];
+        // buffers of the right size from an earlier initialize or batch are kept (allocating,
+        // filling and reading back each instance's on its own took four fifths of a batch of 64)
+        const size_t bytes = sizeof(float) * (size_t)mdp->n;
+        if (registry_holds(vi->d_V, bytes, dev) && registry_holds(vi->d_VPrime, bytes, dev) &&
+                registry_holds(vi->d_pi, bytes, dev)) {
+            sorted_drop(vi->d_V, fn);
+            chunked_drop(vi->d_V, fn);
+            vi->currentHorizon = 0;
+        } else {
+            rc = vi_state_alloc(mdp, vi, fn);
+        }
         ViInst &I = host[b];
         I.n = mdp->n;
         I.m = mdp->m;
@@ -1775,45 +1834,48 @@ int mdp_vi_batch_execute_gpu(const MDP *const *mdps, MDPVIGPU *const *vis, unsig
         I.S = mdp->d_S;
         I.T = mdp->d_T;
         I.R = mdp->d_R;
-        I.V = vis[b]->d_V;
-        I.Vp = vis[b]->d_VPrime;
-        I.pi = vis[b]->d_pi;
-        off[b + 1] = off[b] + I.tiles;
-        maxH = std::max(maxH, I.horizon);
-        if ((size_t)off[b] + I.tiles >= ((size_t)1 << 31))
+        I.V = vi->d_V;
+        I.Vp = vi->d_VPrime;
+        I.pi = vi->d_pi;
+        if ((size_t)off[b] + I.tiles >= ((size_t)1 << 31) ||
+                (size_t)base[b] + I.n >= ((size_t)1 << 31))
             rc = NOVA_ERROR_INVALID_DATA;
+        off[b + 1] = off[b] + I.tiles;
+        base[b + 1] = base[b] + I.n;
+        maxH = std::max(maxH, I.horizon);
     }
     void *mem = nullptr;
-    const size_t bI = up256(sizeof(ViInst) * count), bO = up256(sizeof(unsigned) * (count + 1));
+    const size_t states = base[count];
+    const size_t bI = up256(sizeof(ViInst) * count), bO = up256(sizeof(unsigned) * off.size());
+    const size_t bV = up256(sizeof(float) * states);
     if (rc == NOVA_SUCCESS)
-        rc = device_alloc(&mem, bI + bO, fn, "the batch descriptors");
+        rc = device_alloc(&mem, bI + bO + 2 * bV, fn, "the batch descriptors and values");
     hipStream_t st = stream();
-    hipGraphExec_t exec = nullptr;
+    std::vector<float> values;
+    std::vector<unsigned> actions;
     if (rc == NOVA_SUCCESS) {
-        ViInst *dInst = static_cast<ViInst *>(mem);
-        unsigned *dOff = reinterpret_cast<unsigned *>(static_cast<char *>(mem) + bI);
+        char *c = static_cast<char *>(mem);
+        ViInst *dInst = reinterpret_cast<ViInst *>(c);
+        unsigned *dOff = reinterpret_cast<unsigned *>(c + bI), *dBase = dOff + count + 1;
+        float *dV = reinterpret_cast<float *>(c + bI + bO);
+        unsigned *dPi = reinterpret_cast<unsigned *>(c + bI + bO + bV);
+        values.assign(states, 0.0f);
+        for (unsigned b = 0; b < count; b++)
+            if (vis[b]->VInitial != nullptr)
+                std::memcpy(&values[base[b]], vis[b]->VInitial, sizeof(float) * host[b].n);
         hipError_t e = hipMemcpyAsync(dInst, host.data(), sizeof(ViInst) * count,
                                       hipMemcpyHostToDevice, st);
         if (e == hipSuccess)
-            e = hipMemcpyAsync(dOff, off.data(), sizeof(unsigned) * (count + 1),
+            e = hipMemcpyAsync(dOff, off.data(), sizeof(unsigned) * off.size(),
                                hipMemcpyHostToDevice, st);
         if (e == hipSuccess)
-            e = hipStreamSynchronize(st);
-        hipStream_t cs = capture_stream();
-        hipGraph_t graph = nullptr;
-        if (e == hipSuccess && cs == nullptr)
-            e = hipErrorInvalidValue;
-        if (e == hipSuccess)
-            e = hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal);
+            e = hipMemcpyAsync(dV, values.data(), sizeof(float) * states, hipMemcpyHostToDevice,
+                               st);
+        const dim3 sg((unsigned)((states + kBatchThreads - 1) / kBatchThreads));
         if (e == hipSuccess) {
-            for (unsigned k = 0; k < maxH; k++)
-                hipLaunchKernelGGL(vi_batch_sweep, dim3(off[count]), dim3(kBatchThreads), 0, cs,
-                                   dInst, dOff, count, k);
-            e = hipStreamEndCapture(cs, &graph);
-        }
-        if (e == hipSuccess) {
-            e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-            hipGraphDestroy(graph);
+            hipLaunchKernelGGL(vi_batch_init, sg, dim3(kBatchThreads), 0, st, dInst, dBase, count,
+                               dV);
+            e = hipGetLastError();
         }
         hipEvent_t t0 = nullptr, t1 = nullptr;
         if (e == hipSuccess && elapsedMs) {
@@ -1821,12 +1883,27 @@ int mdp_vi_batch_execute_gpu(const MDP *const *mdps, MDPVIGPU *const *vis, unsig
             hipEventCreate(&t1);
             hipEventRecord(t0, st);
         }
-        if (e == hipSuccess)
-            e = hipGraphLaunch(exec, st);
+        for (unsigned k = 0; k < maxH && e == hipSuccess; k++) {
+            hipLaunchKernelGGL(vi_batch_sweep, dim3(off[count]), dim3(kBatchThreads), 0, st,
+                               dInst, dOff, count, k);
+            e = hipGetLastError();
+        }
         if (e == hipSuccess && elapsedMs)
             hipEventRecord(t1, st);
+        if (e == hipSuccess && policies) {
+            hipLaunchKernelGGL(vi_batch_collect, sg, dim3(kBatchThreads), 0, st, dInst, dBase,
+                               count, dV, dPi);
+            actions.resize(states);
+            e = hipMemcpyAsync(values.data(), dV, sizeof(float) * states, hipMemcpyDeviceToHost,
+                               st);
+            if (e == hipSuccess)
+                e = hipMemcpyAsync(actions.data(), dPi, sizeof(unsigned) * states,
+                                   hipMemcpyDeviceToHost, st);
+        }
+        // (also after an error: the copies above read host memory that ends with this call)
+        const hipError_t es = hipStreamSynchronize(st);
         if (e == hipSuccess)
-            e = hipStreamSynchronize(st);
+            e = es;
         if (elapsedMs) {
             float ms = 0.0f;
             if (e == hipSuccess && t0 && t1)
@@ -1835,16 +1912,21 @@ int mdp_vi_batch_execute_gpu(const MDP *const *mdps, MDPVIGPU *const *vis, unsig
         }
         if (t0) hipEventDestroy(t0);
         if (t1) hipEventDestroy(t1);
-        if (exec)
-            hipGraphExecDestroy(exec);
-        rc = hip_fail(e, fn, "Failed to run the batch graph.", NOVA_ERROR_KERNEL_EXECUTION);
+        rc = hip_fail(e, fn, "Failed to run the batch.", NOVA_ERROR_KERNEL_EXECUTION);
     }
     if (mem)
-        device_free(mem, fn, "the batch descriptors");
+        device_free(mem, fn, "the batch descriptors and values");
     for (unsigned b = 0; b < count && rc == NOVA_SUCCESS; b++) {
         vis[b]->currentHorizon = mdps[b]->horizon;
-        if (policies)
-            rc = mdp_vi_get_policy_gpu(mdps[b], vis[b], &policies[b]);
+        if (policies == nullptr)
+            continue;
+        if (mdp_value_function_initialize(&policies[b], mdps[b]->n, mdps[b]->m, 0) !=
+                NOVA_SUCCESS) {
+            NOVA_ERR(fn, "Could not create the policy.");
+            return NOVA_ERROR_POLICY_CREATION;
+        }
+        std::memcpy(policies[b].V, &values[base[b]], sizeof(float) * mdps[b]->n);
+        std::memcpy(policies[b].pi, &actions[base[b]], sizeof(unsigned) * mdps[b]->n);
     }
     return rc;
 }

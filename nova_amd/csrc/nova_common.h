@@ -28,8 +28,11 @@ constexpr float kHigh = (float)NOVA_FLT_MAX;
 // or on one still holding buffers from an earlier initialize() (its Python wrapper does this,
 // src/mdp/algorithms/mdp_vi_cpu.cpp:112 then leaks them). Only pointers recorded here are
 // released by a repeated initialize().
-void registry_track(const void *p);
+void registry_track(const void *p, size_t bytes = 0, int device = -1);
 bool registry_untrack(const void *p);   // true when p was tracked (and is now forgotten)
+// true when p is tracked as an allocation of exactly `bytes` on this device (so that a repeated
+// initialize of the same size may keep it)
+bool registry_holds(const void *p, size_t bytes, int device);
 
 // new[] that records the allocation.
 template <typename T> T *tracked_new(size_t count)

@@ -61,14 +61,17 @@ int hip_fail(hipError_t e, const char *fn, const char *msg, int code)
 int device_alloc(void **p, size_t bytes, const char *fn, const char *what)
 {
     *p = nullptr;
-    hipError_t e = hipMalloc(p, bytes > 0 ? bytes : 4);
+    int dev = -1;
+    hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess)
+        e = hipMalloc(p, bytes > 0 ? bytes : 4);
     if (e != hipSuccess) {
         *p = nullptr;
         std::fprintf(stderr, "Error[%s]: Failed to allocate device-side memory for %s (%s)\n",
                      fn, what, hipGetErrorString(e));
         return NOVA_ERROR_DEVICE_MALLOC;
     }
-    registry_track(*p);
+    registry_track(*p, bytes, dev);
     return NOVA_SUCCESS;
 }
 

@@ -110,7 +110,7 @@ class MDPValueIterationGPU(_abi.NovaMDPVIGPU):
 
 def batch_execute(solvers, policies=True):
     """Runs mdp_vi_batch_execute_gpu over MDPValueIterationGPU solvers (their MDPs resident on
-    the device): every instance solved as its plain solve would be, all sweeps in one graph.
+    the device): every instance solved as its plain solve would be, one launch per sweep for all.
     Returns (list of (V, pi) or None, device ms)."""
     lib = _abi.load()
     count = len(solvers)

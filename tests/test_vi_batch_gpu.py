@@ -2,6 +2,8 @@
 of every instance in one HIP graph. Each instance must equal the float oracle's run
 (mdp_vi_cpu.cpp:36-63 per sweep) and its plain GPU solve bit for bit, whatever its size,
 horizon (odd, even, 1), gamma, initial values and ragged successor lists."""
+import ctypes as ct
+
 import numpy as np
 import pytest
 
@@ -75,3 +77,31 @@ def test_vi_batch_rejects_wide_action_sets():
     mdp.initialize_gpu()
     with pytest.raises(Exception):
         batch_execute([MDPValueIterationGPU(mdp)])
+
+
+def address(pointer):
+    return ct.cast(pointer, ct.c_void_p).value
+
+
+def test_vi_batch_reuses_and_replaces_buffers():
+    """A second batch over the same solver structs keeps their device buffers (same sizes); after
+    the model behind a struct changes size, it gets new ones. Both equal fresh solves."""
+    batch = uneven(5, 11)
+    objs = solvers(batch)
+    batch_execute(objs)
+    held = [address(s.d_V) for s in objs]
+    res, _ = batch_execute(objs)
+    assert held == [address(s.d_V) for s in objs]
+    other = uneven(5, 12)
+    for s, w in zip(objs, other):
+        s.mdp = MDP.from_arrays(w["S"], w["T"], w["R"], gamma=w["gamma"], horizon=w["horizon"])
+        s.mdp.initialize_gpu()
+        s.mdpPtr = ct.pointer(s.mdp)
+        s._v0 = np.ascontiguousarray(w["V0"])
+        s.VInitial = s._v0.ctypes.data_as(type(s.VInitial))
+    res2, _ = batch_execute(objs)
+    for ws, got in ((batch, res), (other, res2)):
+        for w, (V, pi), s in zip(ws, got, solvers(ws)):
+            pol = s.solve()
+            assert np.array_equal(bits(V), bits(pol.V_array()))
+            assert np.array_equal(pi, pol.pi_array())
