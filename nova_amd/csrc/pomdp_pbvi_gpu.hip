@@ -3323,9 +3323,9 @@ int pomdp_pbvi_initialize_gpu(const POMDP *pomdp, POMDPPBVIGPU *pbvi)
         return rc;
     hipError_t e = hipMemcpy(pbvi->d_Gamma, pbvi->GammaInitial, rn * sizeof(float),
                              hipMemcpyHostToDevice);
-    if (e == hipSuccess)
-        e = hipMemcpy(pbvi->d_GammaPrime, pbvi->GammaInitial, rn * sizeof(float),
-                      hipMemcpyHostToDevice);
+    if (e == hipSuccess)       // (within HBM: the host's copy crosses the link once)
+        e = hipMemcpy(pbvi->d_GammaPrime, pbvi->d_Gamma, rn * sizeof(float),
+                      hipMemcpyDeviceToDevice);
     if (e == hipSuccess)
         e = hipMemset(pbvi->d_pi, 0, pomdp->r * sizeof(unsigned));
     if (e != hipSuccess)
