@@ -169,6 +169,13 @@ __global__ __launch_bounds__(256) void alpha_value_merge(unsigned k, unsigned ti
 // accesses. VEC: rows 16-byte aligned (n % 4 == 0).
 constexpr unsigned kFewAlphas = 16;
 
+// A load at a 32-bit byte offset from a uniform base (one address register a lane)
+template <typename T>
+__device__ __forceinline__ T load_at(const void *base, unsigned bytes)
+{
+    return *reinterpret_cast<const T *>(static_cast<const char *>(base) + bytes);
+}
+
 // PREC: the call's precision, 0 exact, 1 fp32 (each product and sum rounded once, by an FMA), 2
 // operands rounded to bf16 on the way into LDS and fp32 sums.
 template <int X, int CH, bool VEC, int PREC>
@@ -195,14 +202,14 @@ __global__ __launch_bounds__(64) void alpha_value_few(unsigned k, unsigned n, un
 #pragma unroll
         for (int u = 0; u < kPer; u++) {
             const unsigned e = u * 64 + lane;
-            const float *row = rowOf(e / kAcross);
+            // a whole row per load or more: the same row in every lane, addressed from a scalar
+            const float *row = kAcross >= 64 ? rowOf(u * 64 / kAcross) : rowOf(e / kAcross);
             if constexpr (VEC) {
                 const unsigned s = s0 + e % kAcross * 4;
-                pre4[u] = s < n ? *reinterpret_cast<const float4 *>(row + s)
-                                : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                pre4[u] = s < n ? load_at<float4>(row, s * 4u) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             } else {
                 const unsigned s = s0 + e % kAcross;
-                pre[u] = s < n ? row[s] : 0.0f;
+                pre[u] = s < n ? load_at<float>(row, s * 4u) : 0.0f;
             }
         }
     };
@@ -226,7 +233,7 @@ __global__ __launch_bounds__(64) void alpha_value_few(unsigned k, unsigned n, un
         if (s0 + CH < n)
             load(s0 + CH);
         // blocks of 16 states; one belief per lane reads the next block from LDS before it sums
-        // the current one (n = 5,000: 67 -> 62 us; two beliefs per lane lose more to the
+        // the current one (n = 5,000: 67 -> 60 us; two beliefs per lane lose more to the
         // registers this takes, 129 -> 141 us at n = 5,000, r = 1,024, k = 256)
         const unsigned cnt = min((unsigned)CH, (n - s0 + 15) / 16 * 16);
         float4 g[4], bb[X][4];
@@ -358,7 +365,7 @@ void launch_few_of(unsigned few, unsigned k, unsigned n, unsigned r, const float
 // Beliefs per lane of alpha_value_few for a call, or 0 where the mode's own kernel is the faster:
 // one while that gives at most 1,024 waves (one per SIMD), then two, until alpha_value_exact has
 // a workgroup per CU and more. us of a call, 0 / 1 / 2 beliefs per lane: n = 5,000, r = 1,024:
-// k = 4: 602 / 62 / 90; k = 256: 630 / 208 / 131; k = 2,048: 595 / 1,189 / 745. n = 20,000,
+// k = 4: 602 / 60 / 90; k = 256: 630 / 208 / 131; k = 2,048: 595 / 1,189 / 745. n = 20,000,
 // r = 4,096: k = 1: 2,400 / 204 / 311; k = 64: 2,480 / 829 / 460; k = 256: 2,470 / 2,490 /
 // 1,540; k = 512: 2,290 / 4,660 / 3,150. The same line serves fp32, whose GEMM has a workgroup
 // per 256 x 256 block of C (us, the fp32 GEMM / the split GEMM / this: n = 20,000, r = 4,096,
@@ -993,19 +1000,30 @@ int belief_update_rows(const nova::POMDP *pomdp, unsigned k, const float *d_B,
         return rc;
     const unsigned n = pomdp->n, m = pomdp->m;
     // tiles of one action's triples: at most ceil(k / kTileT) + m of them, in chunks whose
-    // state-major beliefs take kTileBytes (and at least a tile per XCD)
-    const bool tiled = update_tiled(k, n, m, pomdp->z);
+    // state-major beliefs take kTileBytes (and at least a tile per XCD; the grid's y extent
+    // bounds them too). Without the memory for a chunk the triples go one by one.
+    bool tiled = update_tiled(k, n, m, pomdp->z);
     const unsigned blocks = (n + kTileS - 1) / kTileS;
     const size_t tileBytes = sizeof(float) * kTileT * (size_t)n;
-    const unsigned maxTiles = tiled ? ((k + kTileT - 1) / kTileT + m + 7) / 8 * 8 : 0;
-    const unsigned chunkTiles =
-        (unsigned)std::min<size_t>(maxTiles, std::max<size_t>(kTileBytes / tileBytes / 8, 1) * 8);
     const size_t normBytes = up256(sizeof(float) * (size_t)k);
     const size_t orderBytes = up256(sizeof(unsigned) * (size_t)k);
-    const size_t listBytes = up256(sizeof(uint4) * (size_t)maxTiles);
+    unsigned maxTiles = ((k + kTileT - 1) / kTileT + m + 7) / 8 * 8;
+    unsigned chunkTiles = (unsigned)std::min<size_t>(
+        std::min(maxTiles, 65528u), std::max<size_t>(kTileBytes / tileBytes / 8, 1) * 8);
+    size_t listBytes = up256(sizeof(uint4) * (size_t)maxTiles);
+    size_t chunkBytes = tileBytes * chunkTiles;
+    if (tiled && g_updateArena.bytes < normBytes + orderBytes + listBytes + chunkBytes) {
+        size_t freeBytes = 0, totalBytes = 0;
+        tiled = hipMemGetInfo(&freeBytes, &totalBytes) == hipSuccess &&
+                freeBytes + g_updateArena.bytes >=
+                    normBytes + orderBytes + listBytes + chunkBytes + ((size_t)64 << 20);
+    }
+    if (!tiled) {
+        maxTiles = chunkTiles = 0;
+        listBytes = chunkBytes = 0;
+    }
     void *mem = nullptr;
-    rc = arena_get(g_updateArena, normBytes + orderBytes + listBytes + tileBytes * chunkTiles, fn,
-                   mem);
+    rc = arena_get(g_updateArena, normBytes + orderBytes + listBytes + chunkBytes, fn, mem);
     if (rc != NOVA_SUCCESS)
         return rc;
     char *c = static_cast<char *>(mem);

@@ -263,7 +263,8 @@ def test_belief_update_batch_bitwise(oracle, n, m, z, ns, k):
 
 @pytest.mark.parametrize("n,m,z,ns,k", [(1, 2, 3, 1, 4100), (130, 3, 5, 4, 4101),
                                         (257, 40, 2, 9, 4200), (8192, 2, 3, 3, 33),
-                                        (8200, 3, 2, 4, 70)])
+                                        (8200, 3, 2, 4, 70),
+                                        (2, 1, 2, 1, 2_100_000)])     # more tiles than a grid's y
 def test_belief_update_tiles_equal_single_triples(oracle, n, m, z, ns, k):
     """Batches that go through tiles of 32 triples (many triples, or n from 8,192 on) against the
     oracle on a sample and against calls below those sizes on every triple: ragged and skewed
@@ -274,7 +275,8 @@ def test_belief_update_tiles_equal_single_triples(oracle, n, m, z, ns, k):
     P = synth.pomdp_arrays(n=n, m=m, z=z, ns=min(ns, n), r=2, rz=1, seed=n + k)
     rng = np.random.default_rng(k)
     S = P["S"].copy()
-    S[rng.random(S.shape[:2]) < 0.2, -1] = -1
+    if n > 2:
+        S[rng.random(S.shape[:2]) < 0.2, -1] = -1
     S[: n // 2, 0, 0] = 0                      # one state with a long predecessor list
     P["S"] = S
     P["O"] = P["O"].copy()
@@ -301,7 +303,7 @@ def test_belief_update_tiles_equal_single_triples(oracle, n, m, z, ns, k):
     got, status = call(0, k)
     assert status[3] == 1 and status[4] == 1 and np.all(got[3:5] == -7.0)
     if n < 8192:
-        step = 1000
+        step = 4000              # (below the tiles' 4,096)
         parts = [call(lo, min(lo + step, k)) for lo in range(0, k, step)]
         assert np.array_equal(bits(got), bits(np.concatenate([x for x, _ in parts])))
         assert np.array_equal(status, np.concatenate([x for _, x in parts]))
