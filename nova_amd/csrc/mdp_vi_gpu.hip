@@ -34,8 +34,9 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr int kTileRows = 2048;   // most (s,a) rows whose Q values a workgroup stages in LDS
-constexpr unsigned kTileRowsSmall = 128, kTileRowsLarge = 512;   // rows per tile (vi_plan)
-constexpr unsigned kTileSpread = 131072;   // models below this many rows take the small tiles
+constexpr unsigned kTileSpread = 131072;   // models below this many rows take 128-row tiles
+constexpr unsigned kTileNarrow = 786432;   // with one entry per lane, below this many 512-row tiles
+constexpr unsigned kTileCUs = 256;         // CUs that one wave of equal tiles is dealt over
 constexpr int kUnroll = 8;        // rows in flight per lane group (8 measured ~4% faster than 4)
 
 typedef int int4v __attribute__((ext_vector_type(4)));
@@ -1410,6 +1411,37 @@ struct ViPlan {
     unsigned grid = 0;
 };
 
+// States per tile of vi_sweep_tiled (wide: four entries per lane).
+//  * Below kTileSpread rows: 128 rows, which spread a small model over the CUs (2,048 rows leave
+//    a 900-state model three workgroups).
+//  * Above: equal tiles of at most kTileRows rows, two or three per CU (four with one entry per
+//    lane, whose lane groups need more rows in flight), all resident at once: tiles of a fixed
+//    size leave a last round that few CUs take part in. One entry per lane below kTileNarrow
+//    rows: 512 rows.
+//  * Beyond what these hold: tiles of two rows per lane group, at least 128 rows. There the
+//    rounds are many, and small tiles mix the loads of one with the sums of another.
+// us per sweep at 2,048 rows / 512 / 128 / the equal tiles, by n, m, ns:
+//   900, 5, 5: 32.5 / 9.8 / 5.4 / -;  10,000, 7, 9: 103 / 27.5 / 9.2 / -;
+//   30,000, 8, 16: 33.7 / 16.4 / 21.5 / 16.3;  80,000, 5, 12: 34.6 / 26.4 / 30.5 / 25.1;
+//   152,347, 5, 12: 51.5 / 52.4 / 54.9 / 46.8;  300,000, 5, 12: 95.0 / 101 / 104 / 95.4;
+//   100,000, 10, 12: 58.6 / 63.0 / 70.2 / 58.1;  200,000, 8, 16: 153 / 136 / 126 / 136;
+//   one entry per lane: 60,000, 12, 3: 20.9 / 12.3 / 16.6 / 13.4;
+//   200,000, 6, 7: 58.8 / 58.4 / 58.5 / 48.4;  180,000, 8, 11: 128 / 117 / 105 / 106
+static unsigned tile_states(unsigned n, unsigned m, unsigned ns, bool wide)
+{
+    const size_t rows = (size_t)n * m;
+    if (rows < (size_t)kTileSpread)
+        return std::max(1u, 128u / m);
+    if (!wide && rows < (size_t)kTileNarrow)
+        return std::max(1u, 512u / m);
+    for (unsigned k = wide ? 2 : 4; k <= (wide ? 3u : 4u); k++) {
+        const unsigned states = (n - 1) / (kTileCUs * k) + 1;
+        if ((size_t)states * m <= (size_t)kTileRows)
+            return states;
+    }
+    return std::max(1u, std::max(128u, 512u / pow2_at_least(wide ? ns / 4 : ns)) / m);
+}
+
 static ViPlan vi_plan(const nova::MDP *mdp, const nova::MDPVIGPU *vi)
 {
     ViPlan p;
@@ -1424,21 +1456,15 @@ static ViPlan vi_plan(const nova::MDP *mdp, const nova::MDPVIGPU *vi)
     const unsigned n = mdp->n, m = mdp->m, ns = mdp->ns;
     const bool aligned = ((reinterpret_cast<uintptr_t>(mdp->d_S) |
                            reinterpret_cast<uintptr_t>(mdp->d_T)) & 15u) == 0;
+    const bool wide = ns % 4 == 0 && aligned && ns <= 256;
     if (m <= (unsigned)kTileRows) {
-        if (ns % 4 == 0 && aligned && ns <= 256)
+        if (wide)
             p.tiled = tiled_for<4>(pow2_at_least(ns / 4));
         else if (ns <= 64)
             p.tiled = tiled_for<1>(pow2_at_least(ns));
     }
     if (p.tiled) {
-        // Small tiles spread a small model over the CUs (at 2,048 rows a 900-state model has three
-        // workgroups); from about two workgroups of 512 rows per CU on, larger tiles keep more
-        // rows of a lane group in flight. us per sweep at 2,048 / 512 / 128 rows:
-        // n = 900, m = 5, ns = 5: 32.5 / 9.8 / 5.4; n = 10,000, m = 7, ns = 9: 103 / 27.5 / 9.2;
-        // n = 30,000, m = 8, ns = 16: 32.6 / 16.6 / 21.2; n = 200,000, m = 6, ns = 7: 58 / 58 / 58
-        const size_t rows = (size_t)n * m;
-        const unsigned tileRows = rows < (size_t)kTileSpread ? kTileRowsSmall : kTileRowsLarge;
-        p.statesPerTile = std::max(1u, tileRows / m);
+        p.statesPerTile = tile_states(n, m, ns, wide);
         p.grid = (n + p.statesPerTile - 1) / p.statesPerTile;
     } else {
         p.grid = (n + kBlock - 1) / kBlock;

@@ -127,6 +127,30 @@ def test_resident_run_vs_oracle(oracle, monkeypatch, n, m, ns, sweeps):
         assert np.array_equal(bits(last), bits(prev))
 
 
+@pytest.mark.parametrize("n,m,ns", [
+    (131071, 1, 4), (131072, 1, 4),          # the last model of small tiles, the first of equal ones
+    (262145, 4, 4), (262144, 4, 4),          # two full tiles of 2,048 rows per CU, and three
+    (393217, 4, 4),                          # past three: tiles by lane group
+    (200, 700, 8), (1500, 2048, 4),          # one or two states per tile; a tile of one state
+    (112347, 7, 3), (112348, 7, 3),          # one entry per lane: 512-row tiles, then equal ones
+    (400001, 5, 3), (420000, 5, 3),          # four equal tiles per CU, and past them
+])
+def test_tile_sizes_vs_oracle(oracle, monkeypatch, n, m, ns):
+    """One sweep of the wave-tiled kernel on both sides of each line of its tile rule."""
+    rng = np.random.default_rng(n)
+    S = rng.integers(0, n, size=(n, m, ns), dtype=np.int32)
+    S[rng.random((n, m)) < 0.2, ns // 2] = -1
+    T = rng.random((n, m, ns), dtype=np.float32) / ns
+    R = np.round(rng.uniform(-1, 1, (n, m)), 1).astype(np.float32)
+    monkeypatch.setenv("NOVA_AMD_VI_KERNEL", "tiled")
+    mdp = MDP.from_arrays(S, T, R, gamma=0.95, horizon=1)
+    mdp.initialize_gpu()
+    v0 = rng.uniform(-5, 5, n).astype(np.float32)
+    V, pi = solve_gpu(mdp, v0)
+    Vo, pio = oracle.vi_run(S, T, R, np.float32(0.95), 1, V0=v0)
+    assert np.array_equal(bits(V), bits(Vo)) and np.array_equal(pi, pio)
+
+
 def test_resident_run_nan_and_infinities(monkeypatch):
     """A NaN at action 0 stays, one at a later action is never taken, all -inf takes action 0:
     the same in the one-launch run and in separate sweeps."""
