@@ -202,15 +202,16 @@ __global__ __launch_bounds__(64) void alpha_value_few(unsigned k, unsigned n, un
 #pragma unroll
         for (int u = 0; u < kPer; u++) {
             const unsigned e = u * 64 + lane;
-            // a whole row per load or more: the same row in every lane, addressed from a scalar
-            const float *row = kAcross >= 64 ? rowOf(u * 64 / kAcross) : rowOf(e / kAcross);
-            if constexpr (VEC) {
-                const unsigned s = s0 + e % kAcross * 4;
-                pre4[u] = s < n ? load_at<float4>(row, s * 4u) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            } else {
-                const unsigned s = s0 + e % kAcross;
-                pre[u] = s < n ? load_at<float>(row, s * 4u) : 0.0f;
-            }
+            // a whole row per load or more: the same row in every lane, addressed from a scalar.
+            // The chunk's start is part of the 64-bit base (rows may pass 4 GB), the lane's 32-bit
+            // offset stays within the chunk.
+            const float *row = (kAcross >= 64 ? rowOf(u * 64 / kAcross) : rowOf(e / kAcross)) + s0;
+            const unsigned in = e % kAcross * (VEC ? 4u : 1u);
+            if constexpr (VEC)
+                pre4[u] = s0 + in < n ? load_at<float4>(row, in * 4u)
+                                      : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            else
+                pre[u] = s0 + in < n ? load_at<float>(row, in * 4u) : 0.0f;
         }
     };
     float acc[X];
@@ -375,9 +376,12 @@ void launch_few_of(unsigned few, unsigned k, unsigned n, unsigned r, const float
 constexpr size_t kFewPairs = 5u << 18;       // most (belief, alpha) pairs, 1.25 Mi
 constexpr unsigned kFewBf16 = 64;
 
-unsigned few_beliefs(unsigned k, unsigned r, int precision)
+constexpr unsigned kFewStates = 1u << 31;    // most states (the kernel's 32-bit state counters)
+
+unsigned few_beliefs(unsigned n, unsigned k, unsigned r, int precision)
 {
     if ((size_t)k * r > kFewPairs || r > 65535u * kFewAlphas ||       // (the grid's y extent)
+            n > kFewStates ||
             (precision == 2 && (k > kFewBf16 || dense_legacy_bf16())))
         return 0;
     const size_t waves = (size_t)((k + 3) / 4) * ((r + kFewAlphas - 1) / kFewAlphas);
@@ -1159,7 +1163,7 @@ extern "C" int nova_amd_alpha_vectors_value_and_action_gpu(unsigned int n, unsig
     }
     std::lock_guard<std::mutex> lock(g_valueMutex);
     hipStream_t st = stream();
-    const unsigned few = few_beliefs(k, r, precision);
+    const unsigned few = few_beliefs(n, k, r, precision);
     const bool exact = precision == 0 || few != 0;       // on the vector ALUs
     const unsigned tileW = exact ? exact_tile(few) : (unsigned)kGT;
     const unsigned colTiles = (r + tileW - 1) / tileW;
@@ -1353,7 +1357,7 @@ extern "C" int nova_amd_alpha_vectors_value_and_action_noalloc_gpu(unsigned int 
     if (c == nullptr)
         return NOVA_ERROR_KERNEL_EXECUTION;
     // the narrower tiles of few beliefs have four times the partials: only where they fit too
-    unsigned few = few_beliefs(k, r, 0);
+    unsigned few = few_beliefs(n, k, r, 0);
     if (few) {
         colTiles = (r + kFewAlphas - 1) / kFewAlphas;
         if (2 * up256(colTiles * k * sizeof(float)) <= kNoAllocScratchBytes)

@@ -99,6 +99,28 @@ def test_exact_few_beliefs_bitwise(oracle, k, n, r, offset):
             assert bits(np.float32(vo)) == bits(Vh[i]) and ao == ah[i] and jo == jh[i], i
 
 
+@pytest.mark.parametrize("extra", [4, 5])        # rows aligned to 16 bytes, or not
+def test_few_beliefs_rows_past_4_gb(extra):
+    """A belief and an alpha of more than 2^30 states: values at both ends of the rows, so that an
+    offset that wraps at 4 GB reads others. The few terms are sums of small integers: exact."""
+    import torch
+    from nova_amd import _abi
+    n = 2 ** 30 + extra
+    B, G = torch.zeros(n, device="cuda"), torch.zeros(n, device="cuda")
+    at = [0, 1, 2, 3, 4, 255, 256, 2 ** 30 - 1, 2 ** 30, 2 ** 30 + 1, n - 1]
+    for x, s in enumerate(at):
+        B[s] = x + 1
+        G[s] = 2 * x + 1
+    pi = torch.full((1,), 3, dtype=torch.int32, device="cuda")
+    V = torch.zeros(1, device="cuda")
+    a = torch.zeros(1, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    assert _abi.load().nova_amd_alpha_vectors_value_and_action_gpu(
+        n, 1, G.data_ptr(), pi.data_ptr(), 1, B.data_ptr(), 0, V.data_ptr(), a.data_ptr(),
+        None) == 0
+    assert float(V) == sum((x + 1) * (2 * x + 1) for x in range(len(at))) and int(a) == 3
+
+
 def test_exact_no_alpha_above_sentinel():
     """Every value at or below -1e10: V = -1e10, action 0 and alpha -1 (the reference leaves
     Vb and a at their initial values). Exact and fp32 only: in bf16 the sentinel itself rounds
