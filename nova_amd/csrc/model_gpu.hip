@@ -59,6 +59,8 @@ template <typename T> static int release_device(T *&p, const char *fn, const cha
 {
     NOVA_AMD_API_LOCK();
     model_changed(transitions);
+    if (transitions)
+        belief_update_release(p);
     int rc = device_free_if_owned(p, fn, what);
     p = nullptr;
     return rc;

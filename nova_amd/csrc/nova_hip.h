@@ -52,6 +52,10 @@ int device_free_if_owned(void *p, const char *fn, const char *what);
 unsigned long long model_generation(bool transitionsOnly);
 void model_changed(bool transitions);
 
+// Releases the predecessor lists and the workspace that belief updates keep between calls, when p
+// is one of the model arrays the lists were built from.
+void belief_update_release(const void *p);
+
 // Checks that every successor index in the valid prefix of each list lies in [0, limit):
 // the kernels gather V[sp]/Gamma[sp] without further checks. Returns the first bad flat index
 // or -1.

@@ -607,20 +607,23 @@ __global__ __launch_bounds__(kTileThreads) void belief_tiles(unsigned n,
 // pass L2: the beliefs, O and the rows written, each as large); 16 triples a tile take 196 us per
 // 48, staging the lists in LDS 160 us (fewer workgroups fit), 8 entries at a time 151 us. Workgroups are dealt to the XCDs
 // in turn: workgroup b takes a tile of XCD b mod 8, so that the workgroups running together on
-// an XCD share one tile's BT.
+// an XCD share one tile's BT (spread = 8; a chunk of fewer than 8 tiles gives each to all XCDs,
+// spread = 1). count tiles of the chunk.
 constexpr unsigned kTileE = 4;
-constexpr size_t kTileBytes = (size_t)128 << 20;     // state-major beliefs of a chunk of tiles
+constexpr size_t kTileBytes = (size_t)128 << 20;     // most state-major beliefs of a chunk of tiles
 
 template <typename IDX>
 __global__ __launch_bounds__(kTileThreads) void belief_update_tiles(unsigned n, unsigned z,
-        unsigned blocks, const uint4 *__restrict__ tiles, const unsigned *__restrict__ order,
+        unsigned blocks, unsigned count, unsigned spread, const uint4 *__restrict__ tiles, const unsigned *__restrict__ order,
         const unsigned *__restrict__ pstart, const IDX *__restrict__ pS,
         const float *__restrict__ pT, const float *__restrict__ O,
         const unsigned *__restrict__ obs, const float *__restrict__ BT, float *__restrict__ Bp)
 {
     __shared__ float buf[kTileT][kTileS + 1];
     __shared__ unsigned row[kTileT];         // the triple's row of Bp, or ~0 when it has none
-    const unsigned b = blockIdx.x / 8, slot = b / blocks * 8 + blockIdx.x % 8;
+    const unsigned b = blockIdx.x / spread, slot = b / blocks * spread + blockIdx.x % spread;
+    if (slot >= count)
+        return;
     const uint4 tile = tiles[slot];
     if (tile.z == 0)
         return;
@@ -842,7 +845,9 @@ struct DenseShape {
 } g_valueShape;
 
 std::mutex g_updateMutex;
-Arena g_updateArena;                 // the normalisers and action order of a batch of belief updates
+// The normalisers, the action order and the tiles of a batch of belief updates: 24 bytes a triple
+// at most and kTileBytes. Given back, as the lists below, with the model (belief_update_release).
+Arena g_updateArena;
 // predecessor lists of the last model seen, keyed by its device arrays
 struct PredLists {
     const void *dS = nullptr, *dT = nullptr, *dO = nullptr;
@@ -971,15 +976,33 @@ static int pred_lists(const nova::POMDP *p, const char *fn)
 
 namespace nova_amd {
 
+// Gives back the belief updates' lists and workspace when an array of the model they were built
+// from is released (the lists are stale from then on).
+void belief_update_release(const void *p)
+{
+    if (p == nullptr)
+        return;
+    std::lock_guard<std::mutex> lock(g_updateMutex);
+    if (g_pred.mem == nullptr || (p != g_pred.dS && p != g_pred.dT && p != g_pred.dO))
+        return;
+    const char *fn = "belief_update_release";
+    device_free(g_pred.mem, fn, "predecessor lists");
+    g_pred = PredLists();
+    device_free(g_updateArena.mem, fn, "policy workspace");
+    g_updateArena = Arena();
+}
+
 // Whether a batch of updates goes through the tiles of kTileT triples: where one workgroup per
 // triple is too slow a walk (n from 8,192 on) or the batch is large, and the actions' groups
 // fill their tiles well enough (a tile costs about the same with 1 triple as with 32). us of a
-// call, workgroup per triple / tiles: n = 20,000, m = 16: k = 128: 796 / 783, k = 1,024:
-// 1,007 / 896, k = 16,384: 6,260 / 3,730; n = 10,000, m = 8: k = 1,024: 306 / 251; n = 3,001,
+// call, workgroup per triple / tiles: n = 20,000, m = 16: k = 1: 770 / 727, k = 33: 815 / 776,
+// k = 128: 796 / 783, k = 1,024: 1,007 / 896, k = 16,384: 6,260 / 3,730; n = 100,000, m = 4:
+// k = 1: 1,550 / 1,060, k = 1,000: 6,920 / 1,860; n = 1,000,000, m = 2: k = 1: 12,000 / 7,780,
+// k = 256: 20,600 / 10,700; n = 10,000, m = 8: k = 1,024: 306 / 251; n = 3,001,
 // m = 7: k = 512: 88 / 99, k = 4,096: 171 / 151; n = 500, m = 4: k = 16,384: 166 / 124.
 static bool update_tiled(unsigned k, unsigned n, unsigned m, unsigned z)
 {
-    if (m > kOrderMaxM || (size_t)n * kTileT * 4 >= ((size_t)1 << 32) ||
+    if (m > kOrderMaxM || (size_t)n * kTileT * 4 > kTileBytes ||
             (size_t)n * z >= ((size_t)1 << 30))      // (32-bit byte offsets)
         return false;
     return (n >= 8192 && (k >= 8 * m || m <= 16)) || (k >= 4096 && k >= 32 * m);
@@ -1003,17 +1026,19 @@ int belief_update_rows(const nova::POMDP *pomdp, unsigned k, const float *d_B,
     if (rc != NOVA_SUCCESS)
         return rc;
     const unsigned n = pomdp->n, m = pomdp->m;
-    // tiles of one action's triples: at most ceil(k / kTileT) + m of them, in chunks whose
-    // state-major beliefs take kTileBytes (and at least a tile per XCD; the grid's y extent
-    // bounds them too). Without the memory for a chunk the triples go one by one.
+    // tiles of one action's triples: at most k and ceil(k / kTileT) + m of them, in chunks whose
+    // state-major beliefs take at most kTileBytes (the grid's y extent bounds them too). Without
+    // the memory for a chunk the triples go one by one.
     bool tiled = update_tiled(k, n, m, pomdp->z);
     const unsigned blocks = (n + kTileS - 1) / kTileS;
     const size_t tileBytes = sizeof(float) * kTileT * (size_t)n;
     const size_t normBytes = up256(sizeof(float) * (size_t)k);
     const size_t orderBytes = up256(sizeof(unsigned) * (size_t)k);
-    unsigned maxTiles = ((k + kTileT - 1) / kTileT + m + 7) / 8 * 8;
-    unsigned chunkTiles = (unsigned)std::min<size_t>(
-        std::min(maxTiles, 65528u), std::max<size_t>(kTileBytes / tileBytes / 8, 1) * 8);
+    unsigned maxTiles = (unsigned)std::min<size_t>(k, ((size_t)k + kTileT - 1) / kTileT + m);
+    unsigned chunkTiles = (unsigned)std::min<size_t>(std::min(maxTiles, 65528u),
+                                                     std::max<size_t>(kTileBytes / tileBytes, 1));
+    if (chunkTiles > 8)
+        chunkTiles = chunkTiles / 8 * 8;
     size_t listBytes = up256(sizeof(uint4) * (size_t)maxTiles);
     size_t chunkBytes = tileBytes * chunkTiles;
     if (tiled && g_updateArena.bytes < normBytes + orderBytes + listBytes + chunkBytes) {
@@ -1022,14 +1047,19 @@ int belief_update_rows(const nova::POMDP *pomdp, unsigned k, const float *d_B,
                 freeBytes + g_updateArena.bytes >=
                     normBytes + orderBytes + listBytes + chunkBytes + ((size_t)64 << 20);
     }
+    void *mem = nullptr;
+    if (tiled && arena_get(g_updateArena, normBytes + orderBytes + listBytes + chunkBytes, fn,
+                           mem) != NOVA_SUCCESS) {
+        (void)hipGetLastError();
+        tiled = false;
+    }
     if (!tiled) {
         maxTiles = chunkTiles = 0;
         listBytes = chunkBytes = 0;
+        rc = arena_get(g_updateArena, normBytes + orderBytes, fn, mem);
+        if (rc != NOVA_SUCCESS)
+            return rc;
     }
-    void *mem = nullptr;
-    rc = arena_get(g_updateArena, normBytes + orderBytes + listBytes + chunkBytes, fn, mem);
-    if (rc != NOVA_SUCCESS)
-        return rc;
     char *c = static_cast<char *>(mem);
     float *norms = reinterpret_cast<float *>(c);
     // without tiles, grouping by action pays only where the predecessor lists exceed an L2
@@ -1043,17 +1073,19 @@ int belief_update_rows(const nova::POMDP *pomdp, unsigned k, const float *d_B,
         hipLaunchKernelGGL(order_by_action, dim3(1), dim3(1024), 0, st, k, m, d_action, order,
                            tiles, maxTiles);
     for (unsigned t0 = 0; t0 < maxTiles; t0 += chunkTiles) {
-        const unsigned cnt = std::min(chunkTiles, maxTiles - t0);      // multiples of 8
+        const unsigned cnt = std::min(chunkTiles, maxTiles - t0);
+        const unsigned spread = cnt >= 8 ? 8 : 1;
+        const dim3 ug(blocks * ((cnt + spread - 1) / spread * spread));
         hipLaunchKernelGGL(belief_tiles, dim3(blocks, cnt), dim3(kTileThreads), 0, st, n,
                            tiles + t0, order, d_rowOf, d_B, BT);
         if (g_pred.pS16 != nullptr)
-            hipLaunchKernelGGL(belief_update_tiles<unsigned short>, dim3(blocks * cnt),
-                               dim3(kTileThreads), 0, st, n, pomdp->z, blocks, tiles + t0, order,
+            hipLaunchKernelGGL(belief_update_tiles<unsigned short>, ug, dim3(kTileThreads), 0, st,
+                               n, pomdp->z, blocks, cnt, spread, tiles + t0, order,
                                g_pred.pstart, g_pred.pS16, g_pred.pT, pomdp->d_O, d_observation,
                                BT, d_Bp);
         else
-            hipLaunchKernelGGL(belief_update_tiles<int>, dim3(blocks * cnt), dim3(kTileThreads),
-                               0, st, n, pomdp->z, blocks, tiles + t0, order, g_pred.pstart,
+            hipLaunchKernelGGL(belief_update_tiles<int>, ug, dim3(kTileThreads), 0, st, n,
+                               pomdp->z, blocks, cnt, spread, tiles + t0, order, g_pred.pstart,
                                g_pred.pS, g_pred.pT, pomdp->d_O, d_observation, BT, d_Bp);
     }
     const int useLds = n <= (unsigned)kUpdLdsFloats ? 1 : 0;

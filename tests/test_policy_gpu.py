@@ -334,6 +334,46 @@ def test_belief_update_tiles_equal_single_triples(oracle, n, m, z, ns, k):
         assert status[i] == rc and np.array_equal(bits(got[i]), bits(bp)), i
 
 
+@pytest.mark.parametrize("n,k", [(1_000_000, 1),      # one tile of 128 MB
+                                 (200_000, 70),       # chunks of five tiles, the last one of three
+                                 (1_048_576, 40), (1_048_577, 3)])   # the largest, and no tiles
+def test_belief_update_of_large_models_takes_bounded_memory(oracle, n, k):
+    """The workspace of an update stays within 128 MiB and the triples' own 24 bytes (beside the
+    predecessor lists), and is given back with the model; results equal the oracle's."""
+    import torch
+    from nova_amd import _abi
+    m, z, ns = 2, 2, 2
+    P = synth.pomdp_arrays(n=n, m=m, z=z, ns=ns, r=2, rz=1, seed=n + k)
+    P["S"] = P["S"].copy()
+    P["S"][:100, 0, 0] = 0
+    p = POMDP.from_dict(P)
+    p.initialize_gpu()
+    rng = np.random.default_rng(k)
+    B = rng.exponential(size=(k, n)).astype(np.float32)
+    B /= B.sum(axis=1, keepdims=True)
+    a = rng.integers(0, m, k).astype(np.int32)
+    o = rng.integers(0, z, k).astype(np.int32)
+    Bt, at, ot = (torch.from_numpy(x).cuda() for x in (B, a, o))
+    out = torch.empty((k, n), device="cuda")
+    st = torch.empty(k, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    assert _abi.load().nova_amd_belief_update_batch_gpu(
+        ct.byref(p), k, Bt.data_ptr(), at.data_ptr(), ot.data_ptr(), out.data_ptr(),
+        st.data_ptr()) == 0
+    lists = 4 * (m * (n + 1) + 2 * n * m * ns + m * z * n)
+    slack = 32 << 20                 # (the driver hands out whole blocks; kernels are loaded)
+    assert before - torch.cuda.mem_get_info()[0] <= lists + (128 << 20) + 24 * k + slack
+    got, status = out.cpu().numpy(), st.cpu().numpy()
+    for i in range(0, k, max(1, k // 8)):
+        rc, bp = oracle.belief_update(P, B[i], int(a[i]), int(o[i]))
+        assert status[i] == rc and np.array_equal(bits(got[i]), bits(bp)), i
+    free = torch.cuda.mem_get_info()[0]
+    model = 4 * (2 * n * m * ns + n * m + m * n * z)
+    p.uninitialize_gpu()
+    assert torch.cuda.mem_get_info()[0] - free >= lists + model - slack
+
+
 def bf16_round(x):
     """float32 -> nearest bfloat16 (ties to even), returned as float32."""
     u = np.asarray(x, np.float32).view(np.uint32).astype(np.uint64)
