@@ -133,14 +133,15 @@ __global__ __launch_bounds__(kVThreads) void alpha_value_exact(unsigned k, unsig
 }
 
 // Merge of the alpha tiles per belief, tile 0 first: V, the winning alpha (or -1) and its
-// action (0 when none beat -1e10, as the reference leaves a).
+// action (0 when none beat -1e10, as the reference leaves a). skip (nullable): when *skip is
+// not 0 the tiles were left out, and there is nothing to merge.
 __global__ __launch_bounds__(256) void alpha_value_merge(unsigned k, unsigned tiles,
         const float *__restrict__ partV, const int *__restrict__ partJ,
         const unsigned *__restrict__ pi, float *__restrict__ V, unsigned *__restrict__ act,
-        int *__restrict__ jOut)
+        int *__restrict__ jOut, const int *__restrict__ skip)
 {
     const unsigned i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= k)
+    if (i >= k || (skip && *skip))
         return;
     float bv = kLow;
     int bj = INT_MAX;
@@ -401,7 +402,7 @@ void launch_exact(unsigned few, int precision, unsigned k, unsigned n, unsigned 
         hipLaunchKernelGGL(alpha_value_exact, dim3((k + kVT - 1) / kVT, tiles), dim3(kVThreads),
                            0, st, k, n, r, B, G, partV, partJ);
         hipLaunchKernelGGL(alpha_value_merge, dim3((k + 255) / 256), dim3(256), 0, st, k, tiles,
-                           partV, partJ, pi, V, act, jOut);
+                           partV, partJ, pi, V, act, jOut, (const int *)nullptr);
         return;
     }
     if (precision == 0)
@@ -1137,10 +1138,11 @@ static int value_split(unsigned n, unsigned r, const float *d_Gamma, const unsig
         if (hipMemGetInfo(&freeBytes, &totalBytes) != hipSuccess ||
                 freeBytes + g_valueArena.bytes < bytes + ((size_t)64 << 20))
             return NOVA_SUCCESS;
-    int rc = arena_get(g_valueArena, bytes, fn, mem);
-    if (rc != NOVA_SUCCESS)
-        return rc;
-    g_valueShape = DenseShape();      // the fp32 layout's padding is overwritten
+    g_valueShape = DenseShape();      // the fp32 layout's padding is overwritten, or released
+    if (arena_get(g_valueArena, bytes, fn, mem) != NOVA_SUCCESS) {
+        (void)hipGetLastError();
+        return NOVA_SUCCESS;
+    }
     char *c = static_cast<char *>(mem);
     int *wild = reinterpret_cast<int *>(c);
     float *partV = reinterpret_cast<float *>(c + 256);
@@ -1160,9 +1162,9 @@ static int value_split(unsigned n, unsigned r, const float *d_Gamma, const unsig
                        (size_t)r * n, gRows, d_Gamma, G, wild);
     hipLaunchKernelGGL(dense_score_split, dim3(rowTiles * colTiles), dim3(kGThreads),
                        kSplitLdsBytes, st, k, r, kpad, rowTiles, colTiles,
-                       (const __bf16 *)A, (const __bf16 *)G, partV, partJ);
+                       (const __bf16 *)A, (const __bf16 *)G, partV, partJ, (const int *)wild);
     hipLaunchKernelGGL(alpha_value_merge, dim3((k + 255) / 256), dim3(256), 0, st, k, colTiles,
-                       partV, partJ, d_pi, d_V, d_action, d_alpha);
+                       partV, partJ, d_pi, d_V, d_action, d_alpha, (const int *)wild);
     if (e == hipSuccess)
         e = hipGetLastError();
     int flag = 0;
@@ -1295,7 +1297,8 @@ extern "C" int nova_amd_alpha_vectors_value_and_action_gpu(unsigned int n, unsig
     }
     if (!exact)
         hipLaunchKernelGGL(alpha_value_merge, dim3((k + 255) / 256), dim3(256), 0, st, k,
-                           colTiles, partV, partJ, d_pi, d_V, d_action, d_alpha);
+                           colTiles, partV, partJ, d_pi, d_V, d_action, d_alpha,
+                           (const int *)nullptr);
     if (e == hipSuccess)
         e = hipGetLastError();
     if (e == hipSuccess)

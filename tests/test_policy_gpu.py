@@ -234,6 +234,39 @@ def test_fp32_operands_without_bf16_parts(odd):
     assert np.all(j[~fine] == 11)
 
 
+def test_fp32_call_with_a_tiny_entry_skips_the_split_gemm():
+    """A belief entry below 2^-100 leaves the call to the fp32 instructions, without the split
+    GEMM's work first: the fp32 GEMM takes about 1.7 times the split one, both together 2.7."""
+    import time
+    import torch
+    from nova_amd import _abi
+    k, n, r = 8192, 4096, 4096
+    g = torch.Generator(device="cuda")
+    g.manual_seed(5)
+    G = torch.rand((r, n), generator=g, device="cuda").mul_(6).sub_(3)
+    B = torch.rand((k, n), generator=g, device="cuda").add_(0.1)
+    pi = torch.zeros(r, dtype=torch.int32, device="cuda")
+    V = torch.empty(k, device="cuda")
+    a = torch.empty(k, dtype=torch.int32, device="cuda")
+
+    def best_of(runs):
+        times = []
+        for _ in range(runs):
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            assert _abi.load().nova_amd_alpha_vectors_value_and_action_gpu(
+                n, r, G.data_ptr(), pi.data_ptr(), k, B.data_ptr(), 1, V.data_ptr(),
+                a.data_ptr(), None) == 0
+            times.append(time.perf_counter() - t)
+        return min(times)
+
+    tame = best_of(8)
+    B[k - 1, n - 1] = 1e-35
+    wild = best_of(8)
+    print("fp32 value/action: %.0f us, with a tiny entry %.0f us" % (tame * 1e6, wild * 1e6))
+    assert wild <= 2.2 * tame
+
+
 def test_large_fp32_against_exact_sample():
     """At n = 20,000 and r = 4,096 (the dense PBVI size) with k = 8,192 beliefs: fp32 against
     exact on the first 256 beliefs (same choice or a near-tie)."""
