@@ -189,8 +189,8 @@ extern "C" int nova_amd_ssp_sweeps_gpu(const MDP *mdp, int absV, const float *d_
 // null, d_alpha (k indices of the chosen alpha, -1 when no alpha beats -1e10, in which case the
 // value is -1e10 and the action 0, as the reference leaves them). precision: 0 = exact (each
 // dot product summed over the states in order with separately rounded products and sums:
-// equal to the reference bit for bit), 1 = fp32 (single-precision products and sums, on the
-// matrix cores for many beliefs), 2 = bf16 operands with fp32 accumulation (the -1e10 sentinel
+// equal to the reference bit for bit), 1 = fp32 (single-precision sums; for many beliefs
+// on the matrix cores, each product of three bf16 parts per operand, within 2^-24 of it), 2 = bf16 operands with fp32 accumulation (the -1e10 sentinel
 // itself rounds to -9.9992e9 there).
 // r <= 4,194,240. Synchronous; calls are serialised.
 extern "C" int nova_amd_alpha_vectors_value_and_action_gpu(unsigned int n, unsigned int r,

@@ -540,12 +540,16 @@ __global__ __launch_bounds__(kGThreads) void dense_score_bf16(unsigned rows, uns
 //
 // An fp32 number is the sum of three bf16 numbers, x = h + m + l (8 significant bits each, every
 // one the rounding of what the earlier ones leave), exactly. Of the nine products of two such
-// sums the six largest, hh, hm, mh, hl, lh and mm, differ from the fp32 product by at most about
-// 2^-26 of it, less than its own rounding, and one bf16 matrix instruction sums sixteen of them
-// per fp32 rounding where the fp32 one sums two. Six bf16 products cost 6/16 of the fp32
-// instruction's time. The split is exact for magnitudes in [2^-100, 2^126] and zero; operands
-// with anything else (dense_split_convert reports it: NaN, infinities, values whose parts
-// would overflow or lose bits to underflow) are left to dense_score<float>. The relative error
+// sums the six largest, hh, hm, mh, hl, lh and mm, are kept. |m| reaches 2^-8 and |l| 2^-17 of
+// the operand, so what the dropped ml, lm and ll hold reaches 2^-24 of the product, one fp32
+// rounding (x = y = 1.0039: 2^-24.0; rms over random operands 2^-27.5): a single product may be
+// off by about 1 ulp, where an fp32 product is off by half of one. From two terms on the sums
+// make up for it: one bf16 matrix instruction sums sixteen products per fp32 rounding, the fp32
+// one two. Six bf16 products cost 6/16 of the fp32 instruction's time. The split is exact for
+// zero and magnitudes in [2^-100, 2^62], whose partial products stay finite too; operands with
+// anything else (dense_split_convert reports it: NaN, infinities, values that lose bits to
+// underflow or whose rounded parts' product could pass the type's range where their own does
+// not) are left to dense_score<float>. The relative error
 // of a row maximum against 64 bits is the smaller here at every size measured: n = 256: 2.0e-7
 // against 2.4e-7, n = 3,000: 6.9e-7 against 7.6e-7, n = 20,000: 1.7e-6 against 2.1e-6 (values
 // within +-3; 1.4e-6 against 2.2e-6 around -20). k = 16,384, r = 4,096, n = 20,000: 20.7 -> 12.1
@@ -564,8 +568,8 @@ constexpr size_t kSplitLdsBytes = (size_t)kSplitStages * 6 * kSplitOp;   // 147,
 // and columns past the data are zeros. *wild is set to 1 when an element cannot be split
 // exactly: dense_score_split and the merge behind it then leave at once, so that a call with one
 // such element costs little more than its fp32 GEMM (k = 8,192, r = n = 4,096: 3,700 us with
-// both run, now 2,440; the fp32 GEMM alone 2,250). Each lane forms two 16-byte chunks of each plane: 8 consecutive k of one row in two
-// neighbouring k blocks.
+// both run, now 2,440; the fp32 GEMM alone 2,250). Each lane forms two 16-byte chunks of each
+// plane: 8 consecutive k of one row in two neighbouring k blocks.
 __global__ __launch_bounds__(kGConvThreads) void dense_split_convert(unsigned n, unsigned kpad,
         size_t count, size_t rowsPad, const float *__restrict__ G, __bf16 *__restrict__ GS,
         int *__restrict__ wild)
@@ -594,7 +598,7 @@ __global__ __launch_bounds__(kGConvThreads) void dense_split_convert(unsigned n,
 #pragma unroll
             for (int e = 0; e < 8; e++) {
                 const float ax = fabsf(x[e]);
-                bad = bad || !(ax == 0.0f || (ax >= 0x1p-100f && ax <= 0x1p126f));
+                bad = bad || !(ax == 0.0f || (ax >= 0x1p-100f && ax <= 0x1p62f));
                 h[e] = (__bf16)x[e];
                 const float r1 = x[e] - (float)h[e];
                 m[e] = (__bf16)r1;

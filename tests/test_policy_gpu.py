@@ -234,6 +234,28 @@ def test_fp32_operands_without_bf16_parts(odd):
     assert np.all(j[~fine] == 11)
 
 
+@pytest.mark.parametrize("x,y", [(1.998 * 2.0 ** 63, 1.9985 * 2.0 ** 63),    # just below the range
+                                 (1.998 * 2.0 ** 120, 1.998 * 2.0 ** 40),    # infinite
+                                 (2.0 ** 62, 1.75 * 2.0 ** 62)])             # one within the split's
+def test_fp32_large_operands(x, y):
+    """Operands whose bf16 parts are finite but whose parts' products are not: the value is the
+    fp32 product's (finite where that is, +infinity otherwise)."""
+    k, n, r = 1400, 70, 1000
+    G, pi, B = instance(k, n, r, seed=4)
+    B[:, 5] = 0.0
+    G[:, 5] = 0.0
+    B[7, 5], G[11, 5] = x, y
+    V, act, j = policy(G, pi).value_and_action_batch(B, "fp32", return_alpha=True)
+    V, j = V.cpu().numpy().astype(np.float64), j.cpu().numpy()
+    with np.errstate(over="ignore"):
+        want = float(np.float32(B[7, 5]) * np.float32(G[11, 5]))
+    assert j[7] == 11 and act.cpu().numpy()[7] == pi[11]
+    assert V[7] == want or abs(V[7] - want) <= 2.0 ** -23 * want
+    rest = np.delete(np.arange(k), 7)
+    C = B.astype(np.float64)[rest] @ G.astype(np.float64).T
+    assert np.all(np.abs(V[rest] - C.max(axis=1)) <= 1e-5 * np.maximum(1.0, np.abs(C.max(axis=1))))
+
+
 def test_fp32_call_with_a_tiny_entry_skips_the_split_gemm():
     """A belief entry below 2^-100 leaves the call to the fp32 instructions, without the split
     GEMM's work first: the fp32 GEMM takes about 1.7 times the split one, both together 2.7."""
