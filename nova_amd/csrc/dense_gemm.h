@@ -549,12 +549,13 @@ __global__ __launch_bounds__(kGThreads) void dense_score_bf16(unsigned rows, uns
 // zero and magnitudes in [2^-100, 2^62], whose partial products stay finite too; operands with
 // anything else (dense_split_convert reports it: NaN, infinities, values that lose bits to
 // underflow or whose rounded parts' product could pass the type's range where their own does
-// not) are left to dense_score<float>. The relative error
-// of a row maximum against 64 bits is the smaller here at every size measured: n = 256: 2.0e-7
-// against 2.4e-7, n = 3,000: 6.9e-7 against 7.6e-7, n = 20,000: 1.7e-6 against 2.1e-6 (values
-// within +-3; 1.4e-6 against 2.2e-6 around -20). k = 16,384, r = 4,096, n = 20,000: 20.7 -> 12.1
-// ms a call, the GEMM 11.1 ms: 1.45 PFLOP/s of bf16 products, 0.58 of the peak (0.50 of it in
-// dense_score_bf16, whose LDS reads per matrix instruction are twice as many).
+// not) are left to dense_score<float>. The relative error of a row maximum against 64 bits is
+// the smaller here at every size measured (values within +-3): n = 50: 4.1e-8 against 1.1e-7,
+// n = 256: 7.9e-8 against 2.3e-7, n = 3,000: 3.0e-7 against 8.3e-7, n = 20,000: 7.5e-7 against
+// 2.1e-6 (7.8e-7 against 2.2e-6 around -20); a row of one nonzero is the exception, 3.3e-8
+// against 2.5e-8. k = 16,384, r = 4,096, n = 20,000: 20.7 -> 12.4 ms a call, the GEMM 11.6 ms:
+// 1.39 PFLOP/s of bf16 products, 0.55 of the peak (0.50 of it in dense_score_bf16, whose LDS
+// reads per matrix instruction are half as many again).
 //
 // Operands lie in the order in which lanes read them from LDS: 1 KB blocks of 32 rows x 16 k,
 // [k / 16][row / 32] with lane 32 c + r's eight k = 8 c .. 8 c + 7 of row r at 16 (32 c + r), per
@@ -618,7 +619,14 @@ __global__ __launch_bounds__(kGConvThreads) void dense_split_convert(unsigned n,
 // jtile * rows + i. 256 x 256 tiles, 8 waves of 128 x 64. Three stages of 16 k lie in LDS. A
 // wave holds a stage's fragments in registers: the smaller planes' are replaced by the next
 // stage's as the products free them, the h fragments alternate between two sets, so LDS reads
-// run behind the 48 matrix instructions of a stage.
+// run behind the 40 matrix instructions of a stage. The hh products follow in a second pass over
+// k, three k blocks of the h planes to a stage: the small products' sums are 2^-7 of the whole,
+// so the roundings of their accumulation do not count, and what is left is one rounding per
+// sixteen hh products. With all six in one pass a block that holds a single nonzero cost six
+// roundings, the fp32 instruction one (rms relative error at n = 1,000, rows of 64 nonzeros:
+// 2.3e-7 in one pass, 4.3e-8 in two, 1.2e-7 with the fp32 instruction; dense rows at n = 20,000:
+// 1.7e-6 and 7.5e-7). The second pass copies a third of the bytes once more: k = 16,384,
+// r = 4,096, n = 20,000: 11.9 -> 12.4 ms a call.
 __global__ __launch_bounds__(kGThreads) void dense_score_split(unsigned rows, unsigned cols,
         unsigned kpad, unsigned rowTiles, unsigned colTiles, const __bf16 *__restrict__ A,
         const __bf16 *__restrict__ B, float *__restrict__ partVal, int *__restrict__ partJ,
@@ -722,7 +730,6 @@ __global__ __launch_bounds__(kGThreads) void dense_score_split(unsigned rows, un
         mul(ah[cur], bm);
         if (more)
             readB(st, 1, bm);
-        mul(ah[cur], bh[cur]);
     };
     for (unsigned ks = 0; ks + 2 < nk; ks += 2) {
         stage(ks, 0, true);
@@ -730,6 +737,59 @@ __global__ __launch_bounds__(kGThreads) void dense_score_split(unsigned rows, un
     }
     stage(nk - 2, 0, true);
     stage(nk - 1, 1, false);
+    __syncthreads();
+
+    // the hh products: stage s holds the h planes' k blocks 3 s, 3 s + 1 and 3 s + 2 (past the
+    // last one: copied again, not multiplied)
+    const unsigned n3 = (nk + 2) / 3;               // at least 2
+    auto issue_h = [&](unsigned s) {
+        unsigned char *st = glds + (size_t)(s % kSplitStages) * 6 * kSplitOp + w * 1024;
+#pragma unroll
+        for (int p = 0; p < 3; p++) {
+            const size_t kb = min(3 * s + p, nk - 1) * (size_t)kSplitBlk;
+            __builtin_amdgcn_global_load_lds((const void *)(As + kb * aRows),
+                                             (void *)(st + p * kSplitOp), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((const void *)(Bs + kb * bRows),
+                                             (void *)(st + (3 + p) * kSplitOp), 16, 0, 0);
+        }
+    };
+    issue_h(0);
+    issue_h(1);
+    issue_h(2);
+    wait_vmem<12>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    readA(glds, 0, al);
+    readB(glds, 0, bh[0]);
+    readA(glds, 1, am);
+    readB(glds, 1, bm);
+    readA(glds, 2, ah[0]);
+    readB(glds, 2, bl);
+    for (unsigned s = 0; s + 1 < n3; s++) {
+        mul(al, bh[0]);
+        const unsigned char *st = glds + (size_t)((s + 1) % kSplitStages) * 6 * kSplitOp;
+        if (s + 2 < n3)
+            asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)" ::: "memory");
+        else
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (s + 3 < n3)
+            issue_h(s + 3);
+        readA(st, 0, al);
+        readB(st, 0, bh[0]);
+        mul(am, bm);
+        readA(st, 1, am);
+        readB(st, 1, bm);
+        mul(ah[0], bl);
+        readA(st, 2, ah[0]);
+        readB(st, 2, bl);
+    }
+    mul(al, bh[0]);
+    if (3 * n3 - 2 < nk)
+        mul(am, bm);
+    if (3 * n3 - 1 < nk)
+        mul(ah[0], bl);
     __syncthreads();
 
     // epilogue: per row, the first maximiser over this tile's 256 columns

@@ -256,6 +256,30 @@ def test_fp32_large_operands(x, y):
     assert np.all(np.abs(V[rest] - C.max(axis=1)) <= 1e-5 * np.maximum(1.0, np.abs(C.max(axis=1))))
 
 
+@pytest.mark.parametrize("nonzeros", [4, 16, 64])
+def test_fp32_split_is_no_less_precise_on_sparse_beliefs(nonzeros):
+    """Beliefs of a few nonzeros among 1,000 states: the split GEMM's rms error against FP64 is at
+    most that of one FMA per product in order (the calls of few beliefs, whose sums are those of
+    the fp32 matrix instruction bit for bit)."""
+    import torch
+    k, n, r = 4096, 1000, 512
+    rng = np.random.default_rng(nonzeros)
+    G = rng.uniform(-3, 3, (r, n)).astype(np.float32)
+    pi = rng.integers(0, 5, r).astype(np.uint32)
+    B = np.zeros((k, n))
+    at = rng.random((k, n)).argsort(axis=1)[:, :nonzeros]
+    np.put_along_axis(B, at, rng.exponential(size=(k, nonzeros)), axis=1)
+    B = (B / B.sum(axis=1, keepdims=True)).astype(np.float32)
+    best = (B.astype(np.float64) @ G.astype(np.float64).T).max(axis=1)
+    p = policy(G, pi)
+    V = p.value_and_action_batch(B, "fp32")[0].cpu().numpy()
+    chain = torch.cat([p.value_and_action_batch(B[q:q + 2048], "fp32")[0]
+                       for q in range(0, k, 2048)]).cpu().numpy()       # 1 Mi pairs each
+    rms = [float(np.sqrt(np.mean(((x - best) / best) ** 2))) for x in (V, chain)]
+    print("sparse beliefs, %d nonzeros: split %.3g, one FMA per product %.3g" % (nonzeros, *rms))
+    assert rms[0] <= rms[1]
+
+
 def test_fp32_call_with_a_tiny_entry_skips_the_split_gemm():
     """A belief entry below 2^-100 leaves the call to the fp32 instructions, without the split
     GEMM's work first: the fp32 GEMM takes about 1.7 times the split one, both together 2.7."""
