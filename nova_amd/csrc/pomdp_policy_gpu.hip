@@ -178,8 +178,9 @@ __device__ __forceinline__ T load_at(const void *base, unsigned bytes)
 }
 
 // PREC: the call's precision, 0 exact, 1 fp32 (each product and sum rounded once, by an FMA), 2
-// operands rounded to bf16 on the way into LDS and fp32 sums.
-template <int X, int CH, bool VEC, int PREC>
+// operands rounded to bf16 on the way into LDS and fp32 sums. FAR: rows of more than 2^30 states
+// (VEC rows are addressed that way at any size; without VEC it takes a tenth longer).
+template <int X, int CH, bool VEC, int PREC, bool FAR>
 __global__ __launch_bounds__(64) void alpha_value_few(unsigned k, unsigned n, unsigned r,
         const float *__restrict__ B, const float *__restrict__ G, float *__restrict__ partV,
         int *__restrict__ partJ)
@@ -204,15 +205,16 @@ __global__ __launch_bounds__(64) void alpha_value_few(unsigned k, unsigned n, un
         for (int u = 0; u < kPer; u++) {
             const unsigned e = u * 64 + lane;
             // a whole row per load or more: the same row in every lane, addressed from a scalar.
-            // The chunk's start is part of the 64-bit base (rows may pass 4 GB), the lane's 32-bit
-            // offset stays within the chunk.
-            const float *row = (kAcross >= 64 ? rowOf(u * 64 / kAcross) : rowOf(e / kAcross)) + s0;
-            const unsigned in = e % kAcross * (VEC ? 4u : 1u);
+            // FAR: the chunk's start is part of the 64-bit base, as a 32-bit offset from the row's
+            // start would wrap at 4 GB.
+            const float *row = (kAcross >= 64 ? rowOf(u * 64 / kAcross) : rowOf(e / kAcross)) +
+                               (FAR ? s0 : 0u);
+            const unsigned in = e % kAcross * (VEC ? 4u : 1u), at = FAR ? in : s0 + in;
             if constexpr (VEC)
-                pre4[u] = s0 + in < n ? load_at<float4>(row, in * 4u)
+                pre4[u] = s0 + in < n ? load_at<float4>(row, at * 4u)
                                       : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             else
-                pre[u] = s0 + in < n ? load_at<float>(row, in * 4u) : 0.0f;
+                pre[u] = s0 + in < n ? load_at<float>(row, at * 4u) : 0.0f;
         }
     };
     float acc[X];
@@ -347,11 +349,14 @@ void launch_few(unsigned k, unsigned n, unsigned r, const float *B, const float 
                                      reinterpret_cast<uintptr_t>(G)) & 15u) == 0;
     const dim3 g((k + 4 * X - 1) / (4 * X), (r + kFewAlphas - 1) / kFewAlphas);
     if (vec)
-        hipLaunchKernelGGL((alpha_value_few<X, CH, true, PREC>), g, dim3(64), 0, st, k, n, r, B,
-                           G, partV, partJ);
+        hipLaunchKernelGGL((alpha_value_few<X, CH, true, PREC, true>), g, dim3(64), 0, st, k, n, r,
+                           B, G, partV, partJ);
+    else if (n <= 1u << 30)
+        hipLaunchKernelGGL((alpha_value_few<X, CH, false, PREC, false>), g, dim3(64), 0, st, k, n,
+                           r, B, G, partV, partJ);
     else
-        hipLaunchKernelGGL((alpha_value_few<X, CH, false, PREC>), g, dim3(64), 0, st, k, n, r, B,
-                           G, partV, partJ);
+        hipLaunchKernelGGL((alpha_value_few<X, CH, false, PREC, true>), g, dim3(64), 0, st, k, n, r,
+                           B, G, partV, partJ);
 }
 
 template <int PREC>
