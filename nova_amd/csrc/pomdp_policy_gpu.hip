@@ -178,8 +178,10 @@ __device__ __forceinline__ T load_at(const void *base, unsigned bytes)
 }
 
 // PREC: the call's precision, 0 exact, 1 fp32 (each product and sum rounded once, by an FMA), 2
-// operands rounded to bf16 on the way into LDS and fp32 sums. FAR: rows of more than 2^30 states
-// (VEC rows are addressed that way at any size; without VEC it takes a tenth longer).
+// operands rounded to bf16 on the way into LDS and fp32 sums of 16 products at a time, as the
+// bf16 matrix instruction takes them (a chain of single products is 2.4 times as far from 64
+// bits: n = 20,000: 1.8e-6 against 5.9e-7, the matrix instruction 7.2e-7). FAR: rows of more than
+// 2^30 states (VEC rows are addressed that way at any size; without VEC it takes a tenth longer).
 template <int X, int CH, bool VEC, int PREC, bool FAR>
 __global__ __launch_bounds__(64) void alpha_value_few(unsigned k, unsigned n, unsigned r,
         const float *__restrict__ B, const float *__restrict__ G, float *__restrict__ partV,
@@ -252,6 +254,10 @@ __global__ __launch_bounds__(64) void alpha_value_few(unsigned k, unsigned n, un
             }
         };
         auto sum = [&](const float4 (&gq)[4], const float4 (&bq)[X][4]) {
+            float part[X];
+#pragma unroll
+            for (int x = 0; x < X; x++)
+                part[x] = PREC == 2 ? 0.0f : acc[x];
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 const float g4[4] = {gq[v].x, gq[v].y, gq[v].z, gq[v].w};
@@ -260,10 +266,13 @@ __global__ __launch_bounds__(64) void alpha_value_few(unsigned k, unsigned n, un
 #pragma unroll
                     for (int x = 0; x < X; x++) {
                         const float b4[4] = {bq[x][v].x, bq[x][v].y, bq[x][v].z, bq[x][v].w};
-                        acc[x] = PREC == 0 ? __fadd_rn(acc[x], __fmul_rn(g4[e], b4[e]))
-                                           : __fmaf_rn(g4[e], b4[e], acc[x]);
+                        part[x] = PREC == 0 ? __fadd_rn(part[x], __fmul_rn(g4[e], b4[e]))
+                                            : __fmaf_rn(g4[e], b4[e], part[x]);
                     }
             }
+#pragma unroll
+            for (int x = 0; x < X; x++)
+                acc[x] = PREC == 2 ? __fadd_rn(acc[x], part[x]) : part[x];
         };
         if constexpr (X == 1) {
             read(0, g, bb);

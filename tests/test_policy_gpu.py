@@ -191,6 +191,23 @@ def test_few_beliefs_fp32_and_bf16(k, n, r, prec):
     assert np.array_equal(act, pi[j])
 
 
+@pytest.mark.parametrize("n,r", [(100, 600), (1000, 600), (4999, 1200), (20000, 600)])
+def test_bf16_few_beliefs_are_as_precise_as_the_matrix_cores(n, r):
+    """bf16 calls of at most 64 beliefs and calls of more: the rms error of the sums against FP64
+    (over the rounded operands) is no larger on the vector ALUs."""
+    import torch
+    k = 256
+    G, pi, B = instance(k, n, r, seed=n + r)
+    p = policy(G, pi)
+    best = (bf16_round(B).astype(np.float64) @ bf16_round(G).astype(np.float64).T).max(axis=1)
+    gemm = p.value_and_action_batch(B, "bf16")[0].cpu().numpy()
+    few = torch.cat([p.value_and_action_batch(B[q:q + 64], "bf16")[0]
+                     for q in range(0, k, 64)]).cpu().numpy()
+    rms = [float(np.sqrt(np.mean((x - best) ** 2) / np.mean(best ** 2))) for x in (few, gemm)]
+    print("bf16 sums, n=%d: few %.3g, GEMM %.3g" % (n, *rms))
+    assert rms[0] <= rms[1]
+
+
 # more than 1.25 Mi (belief, alpha) pairs: the split GEMM
 @pytest.mark.parametrize("k,n,r", [(1300, 1, 1100), (1025, 64, 1300), (5200, 130, 257),
                                    (700, 1000, 2000)])
