@@ -388,15 +388,26 @@ void launch_few_of(unsigned few, unsigned k, unsigned n, unsigned r, const float
 // k = 16: 5,140 / 2,310 / 214; k = 256: 5,150 / 2,320 / 1,510; n = 1,000, r = 200, k = 4,096:
 // 315 / 177 / 82). bf16 calls take it up to kFewBf16 beliefs (n = 20,000, r = 4,096: k = 8: 213,
 // k = 64: 408 against 508 of the bf16 GEMM at any k up to 256).
+// Short rows leave nothing to spread: exact calls of at most kFewShort states, and of many
+// pairs (kFewShortPairs) in both directions, keep the square tiles (n = 50: k = 1,000, r = 1,200: 34 / 34;
+// k = 18,750, r = 64: 29 / 34; k = 50,000, r = 20: 34 / 38; k = 9,375, r = 64: 29 / 28;
+// k = 75,000, r = 16: 40 / 34; n = 100: k = 18,750, r = 64: 38 / 34).
+// The partials of k >= kMergeWaves beliefs (at most 10 tiles each) are merged a lane per belief,
+// fewer a wave per belief (us of a call, wave / lane: n = 50, k = 50,000, r = 20: 49 / 38;
+// k = 8,192, r = 10: 24 / 22; k = 4,096, r = 300: 36 / 40).
 constexpr size_t kFewPairs = 5u << 18;       // most (belief, alpha) pairs, 1.25 Mi
+constexpr size_t kFewShortPairs = 9u << 16;  // of short rows
+constexpr unsigned kFewShort = 64;
 constexpr unsigned kFewBf16 = 64;
-
 constexpr unsigned kFewStates = 1u << 31;    // most states (the kernel's 32-bit state counters)
+constexpr unsigned kMergeWaves = 8192;
 
 unsigned few_beliefs(unsigned n, unsigned k, unsigned r, int precision)
 {
     if ((size_t)k * r > kFewPairs || r > 65535u * kFewAlphas ||       // (the grid's y extent)
             n > kFewStates ||
+            (precision == 0 && n <= kFewShort && (size_t)k * r > kFewShortPairs && k >= 1024 &&
+             r > kFewAlphas) ||
             (precision == 2 && (k > kFewBf16 || dense_legacy_bf16())))
         return 0;
     const size_t waves = (size_t)((k + 3) / 4) * ((r + kFewAlphas - 1) / kFewAlphas);
@@ -425,8 +436,12 @@ void launch_exact(unsigned few, int precision, unsigned k, unsigned n, unsigned 
         launch_few_of<1>(few, k, n, r, B, G, partV, partJ, st);
     else
         launch_few_of<2>(few, k, n, r, B, G, partV, partJ, st);
-    hipLaunchKernelGGL(alpha_value_merge_few, dim3(k), dim3(64), 0, st, k, tiles, partV, partJ,
-                       pi, V, act, jOut);
+    if (k < kMergeWaves)
+        hipLaunchKernelGGL(alpha_value_merge_few, dim3(k), dim3(64), 0, st, k, tiles, partV, partJ,
+                           pi, V, act, jOut);
+    else
+        hipLaunchKernelGGL(alpha_value_merge, dim3((k + 255) / 256), dim3(256), 0, st, k, tiles,
+                           partV, partJ, pi, V, act, jOut, (const int *)nullptr);
 }
 
 __global__ __launch_bounds__(256) void fill_ones(unsigned count, float *__restrict__ x)

@@ -99,6 +99,48 @@ def test_exact_few_beliefs_bitwise(oracle, k, n, r, offset):
             assert bits(np.float32(vo)) == bits(Vh[i]) and ao == ah[i] and jo == jh[i], i
 
 
+@pytest.mark.parametrize("k,n,r,offset", [
+    (1300, 97, 1100, 0), (1300, 257, 1100, 1), (2600, 32, 600, 0),     # above 1.25 Mi pairs
+    (1024, 64, 641, 0), (1024, 65, 641, 0),      # short rows above 576 Ki pairs, and one state more
+    (1023, 64, 641, 0), (41_000, 7, 16, 0), (41_000, 7, 17, 0),        # too few in one direction
+    (8191, 20, 70, 0), (8192, 20, 70, 0), (8192, 65, 70, 0),           # either merge
+])
+def test_exact_square_tiles_and_few_beliefs_at_their_limits(oracle, k, n, r, offset):
+    """Both sides of the rules between the 64 x 64 tiles and the one-wave tiles, with rows of one
+    step of 32 states and of several, full and ragged, through both entries."""
+    test_exact_few_beliefs_bitwise(oracle, k, n, r, offset)
+
+
+def test_exact_calls_of_many_beliefs_and_few_alphas_keep_their_time():
+    """1,000,000 (belief, alpha) pairs of 50 states cost no more than 1,320,000: the call must not
+    spend its time in a wave per belief that merges two partials."""
+    import time
+    import torch
+    from nova_amd import _abi
+
+    def best_of(k, r, runs=60):
+        g = torch.Generator(device="cuda")
+        g.manual_seed(k)
+        G = torch.rand((r, 50), generator=g, device="cuda")
+        B = torch.rand((k, 50), generator=g, device="cuda")
+        pi = torch.zeros(r, dtype=torch.int32, device="cuda")
+        V = torch.empty(k, device="cuda")
+        a = torch.empty(k, dtype=torch.int32, device="cuda")
+        times = []
+        for _ in range(runs):
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            assert _abi.load().nova_amd_alpha_vectors_value_and_action_gpu(
+                50, r, G.data_ptr(), pi.data_ptr(), k, B.data_ptr(), 0, V.data_ptr(),
+                a.data_ptr(), None) == 0
+            times.append(time.perf_counter() - t)
+        return min(times)
+
+    fewer, more = best_of(50_000, 20), best_of(40_000, 33)
+    print("exact value/action: 1.00 M pairs %.1f us, 1.32 M %.1f us" % (fewer * 1e6, more * 1e6))
+    assert fewer <= 1.2 * more
+
+
 @pytest.mark.parametrize("extra", [4, 5])        # rows aligned to 16 bytes, or not
 def test_few_beliefs_rows_past_4_gb(extra):
     """A belief and an alpha of more than 2^30 states: values at both ends of the rows, so that an
