@@ -1419,7 +1419,10 @@ struct ViPlan {
 //    size leave a last round that few CUs take part in. One entry per lane below kTileNarrow
 //    rows: 512 rows.
 //  * Beyond what these hold: tiles of two rows per lane group, at least 128 rows. There the
-//    rounds are many, and small tiles mix the loads of one with the sums of another.
+//    rounds are many, and small tiles mix the loads of one with the sums of another. With many
+//    actions 24 / ns states or more: a state's maximum over its actions is one lane's chain,
+//    while the other lanes of a tile of few states wait (n = 10,500, m = 200, ns = 2: 36.9 us a
+//    sweep with one state, 23.9 with five, 26.6 with ten; ns = 16: 108 with one, 123 with five).
 // us per sweep at 2,048 rows / 512 / 128 / the equal tiles, by n, m, ns:
 //   900, 5, 5: 32.5 / 9.8 / 5.4 / -;  10,000, 7, 9: 103 / 27.5 / 9.2 / -;
 //   30,000, 8, 16: 33.7 / 16.4 / 21.5 / 16.3;  80,000, 5, 12: 34.6 / 26.4 / 30.5 / 25.1;
@@ -1439,7 +1442,8 @@ static unsigned tile_states(unsigned n, unsigned m, unsigned ns, bool wide)
         if ((size_t)states * m <= (size_t)kTileRows)
             return states;
     }
-    return std::max(1u, std::max(128u, 512u / pow2_at_least(wide ? ns / 4 : ns)) / m);
+    const unsigned least = std::min((unsigned)kTileRows / m, std::max(1u, 24u / ns));
+    return std::max(least, std::max(128u, 512u / pow2_at_least(wide ? ns / 4 : ns)) / m);
 }
 
 static ViPlan vi_plan(const nova::MDP *mdp, const nova::MDPVIGPU *vi)

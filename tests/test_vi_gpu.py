@@ -363,3 +363,17 @@ def test_layouts_rebuilt_with_other_settings(oracle, monkeypatch):
             V, pi = vi.device_values()
             assert np.array_equal(bits(V), bits(Vo)) and np.array_equal(pi, pio), setting
         del vi
+
+
+def test_sweeps_with_many_actions_keep_their_time():
+    """2,100,000 rows of 200 actions a state sweep no slower than of 16: tiles of few states would
+    leave most lanes waiting for one lane's maximum over the actions."""
+    times = {}
+    for n, m in ((10_500, 200), (131_250, 16)):
+        w = synth.mdp_arrays(n=n, m=m, ns=2, seed=1, gamma=0.95, horizon=10)
+        mdp = MDP.from_arrays(w["S"], w["T"], w["R"], gamma=w["gamma"], horizon=10)
+        mdp.initialize_gpu()
+        vi = MDPValueIterationGPU(mdp, Vinitial=np.zeros(n, np.float32))
+        times[m] = min(vi.run(40) for _ in range(8)) / 40 * 1e3
+    print("us a sweep: m = 200: %.1f, m = 16: %.1f" % (times[200], times[16]))
+    assert times[200] <= 1.12 * times[16]
