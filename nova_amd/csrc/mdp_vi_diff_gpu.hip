@@ -581,7 +581,11 @@ static void sweep64(const nova::MDP *mdp, const double *Va, double *Vb, unsigned
     const unsigned G = std::min(64u, pow2_at_least_u(std::min(mdp->ns, 64u)));
     // rows per workgroup: enough workgroups that eight waves a SIMD hide the gathers' latency
     // (n = 200,000, m = 8, ns = 16: 147 us a sweep at 1,024 rows, 137 at 256, 130 at 128)
-    const unsigned spt = std::max(1u, 128u / mdp->m);
+    // With many actions 24 / ns states or more, within 1,024 rows: one lane per state takes the
+    // maximum over its actions, and a workgroup of few states leaves the others idle meanwhile
+    // (n = 36,839, m = 200, ns = 2: 131 us a sweep with one state a workgroup, 84 with five).
+    const unsigned least = std::min(1024u / mdp->m, std::max(1u, 24u / mdp->ns));
+    const unsigned spt = std::max(std::max(1u, least), 128u / mdp->m);
     const unsigned grid = (mdp->n + spt - 1) / spt;
     const double gamma = (double)mdp->gamma;
 #define NOVA_SW64(GG)                                                                        \

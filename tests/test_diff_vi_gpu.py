@@ -208,3 +208,21 @@ def test_finite_differences_full_size():
           "the step of an action tie, %d with one-sided slopes apart)" % (max(errs), skipped,
                                                                            kinked))
     assert max(errs) <= 1e-3
+
+
+def test_fp64_sweeps_with_many_actions_keep_their_time():
+    """The same for the FP64 sweeps of a solve (7,368,000 rows, time per sweep of a solve)."""
+    import time
+    per = {}
+    for n, m in ((36_840, 200), (460_500, 16)):
+        R, T, S = tensors(synth.mdp_arrays(n=n, m=m, ns=2, seed=1, gamma=0.9))
+        best = np.inf
+        for _ in range(5):
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            sweeps = solve(R, T, S, 0.9, tol=1e-10)[2]
+            torch.cuda.synchronize()
+            best = min(best, (time.perf_counter() - t) / sweeps)
+        per[m] = best * 1e6
+    print("us a sweep of a solve: m = 200: %.1f, m = 16: %.1f" % (per[200], per[16]))
+    assert per[200] <= 1.12 * per[16]
