@@ -89,58 +89,60 @@ __global__ __launch_bounds__(kB) void mu_init(unsigned n, unsigned rz, const int
     }
 }
 
-// u[i][s'] = sum over predecessors (s, l) of s' under a_i of T(s,a_i,l) mu[i][s], one workgroup per
-// alpha with mu[i] in LDS where it fits (useLds), a lane's list entries requested kPredBatch at
-// a time. One entry at a time with mu gathered from L2, each lane was a chain of two loads per
-// entry: 220 us for r = 1,024, n = 5,000, ns = 8, now 107 us.
-constexpr unsigned kPredThreads = 1024;
-constexpr unsigned kPredBatch = 8;
+// u[i][s'] = sum over predecessors (s, l) of s' under a_i of T(s,a_i,l) mu[i][s] (alpha i is
+// blockIdx.y), a lane's list entries requested BATCH at a time. LDS: one workgroup per alpha with
+// mu[i] in LDS, where it fits and the alphas fill the chip; otherwise one lane per state, mu
+// gathered from L2, an alpha's workgroups side by side so that its row stays there. One entry at
+// a time, each lane was a chain of two loads per entry: 220 us for r = 1,024, n = 5,000, ns = 8,
+// now 107 us. us of a replay of 20 steps, one entry at a time / LDS / gathered: n = 5,000, ns = 8:
+// r = 8: 922 / 1,385 / 893, r = 200: 2,450 / 2,184 / 2,226, r = 1,024: 8,170 / 5,970 / 7,200;
+// ns = 2, r = 200: 1,554 / 1,615 / 1,528; n = 20,000, r = 64: 3,890 / 4,670 / 3,560; n = 30,000,
+// r = 2: 2,790 / 5,930 / 2,720.
+constexpr unsigned kPredThreads = 1024;          // lanes with mu in LDS (kB without)
 constexpr unsigned kPredLds = 36 * 1024;         // states of mu in LDS (144 KB)
+constexpr unsigned kPredAlphas = 256;            // fewest alphas with mu in LDS
 
-__global__ __launch_bounds__(kPredThreads) void pred_gather(unsigned n,
+template <bool LDS, unsigned BATCH>
+__global__ __launch_bounds__(LDS ? kPredThreads : kB) void pred_gather(unsigned n,
         const int *__restrict__ act, const unsigned *__restrict__ pstart,
         const int *__restrict__ pS, const float *__restrict__ pT, const float *__restrict__ mu,
-        float *__restrict__ u, int useLds)
+        float *__restrict__ u)
 {
     extern __shared__ float row[];
-    const unsigned i = blockIdx.x, t = threadIdx.x;
+    constexpr unsigned kLanes = LDS ? kPredThreads : kB;
+    const unsigned i = blockIdx.y, t = threadIdx.x;
+    const unsigned first = blockIdx.x * kLanes + t, step = gridDim.x * kLanes;
     const int a = act[i];
     const float *mi = mu + (size_t)i * n;
     float *ui = u + (size_t)i * n;
     if (a < 0) {
-        for (unsigned sp = t; sp < n; sp += kPredThreads)
+        for (unsigned sp = first; sp < n; sp += step)
             ui[sp] = 0.0f;
         return;
     }
-    if (useLds) {
-        for (unsigned s = t; s < n; s += kPredThreads)
+    if constexpr (LDS) {
+        for (unsigned s = t; s < n; s += kLanes)
             row[s] = mi[s];
         __syncthreads();
     }
     const unsigned *ps = pstart + (size_t)a * (n + 1);
-    for (unsigned sp = t; sp < n; sp += kPredThreads) {
+    for (unsigned sp = first; sp < n; sp += step) {
         const unsigned lo = ps[sp], hi = ps[sp + 1];
         float acc = 0.0f;
-        for (unsigned q0 = lo; q0 < hi; q0 += kPredBatch) {
-            int si[kPredBatch];
-            float tv[kPredBatch];
+        for (unsigned q0 = lo; q0 < hi; q0 += BATCH) {
+            int si[BATCH];
+            float tv[BATCH];
 #pragma unroll
-            for (unsigned e = 0; e < kPredBatch; e++) {
+            for (unsigned e = 0; e < BATCH; e++) {
                 const unsigned q = min(q0 + e, hi - 1);
                 si[e] = pS[q];
                 tv[e] = pT[q];
             }
-            if (useLds) {
 #pragma unroll
-                for (unsigned e = 0; e < kPredBatch; e++)
-                    tv[e] = tv[e] * row[si[e]];
-            } else {
+            for (unsigned e = 0; e < BATCH; e++)
+                tv[e] = tv[e] * (LDS ? row[si[e]] : mi[si[e]]);
 #pragma unroll
-                for (unsigned e = 0; e < kPredBatch; e++)
-                    tv[e] = tv[e] * mi[si[e]];
-            }
-#pragma unroll
-            for (unsigned e = 0; e < kPredBatch; e++)
+            for (unsigned e = 0; e < BATCH; e++)
                 acc = q0 + e < hi ? acc + tv[e] : acc;
         }
         ui[sp] = acc;
@@ -433,16 +435,20 @@ int pomdp_pbvi_replay_grad_gpu(const POMDP *pomdp, unsigned int iterations, cons
         hipLaunchKernelGGL(mu_init, dim3(r), dim3(kB), 0, st, n, pomdp->rz, pomdp->d_Z,
                            pomdp->d_B, dfs, dfl, muA);
         const dim3 g((n + kB - 1) / kB, r), ga((n + kB - 1) / kB, m);
-        const int predLds = n <= kPredLds ? 1 : 0;
-        hipFuncSetAttribute((const void *)pred_gather,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, 4 * kPredLds);
+        const bool predLds = n <= kPredLds && r >= kPredAlphas &&
+                             hipFuncSetAttribute((const void *)pred_gather<true, 8>,
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                 4 * kPredLds) == hipSuccess;
         for (int t = (int)H - 1; t >= 0; t--) {
             const int *act = d_recA + (size_t)t * r;
             hipLaunchKernelGGL(dr_accumulate, ga, dim3(kB), 0, st, n, m,
                                das + (size_t)t * (m + 1), dal, muA, d_dR);
-            hipLaunchKernelGGL(pred_gather, dim3(r), dim3(kPredThreads),
-                               predLds ? sizeof(float) * n : 0, st, n, act, dps, dpS, dpT, muA, u,
-                               predLds);
+            if (predLds)
+                hipLaunchKernelGGL((pred_gather<true, 8>), dim3(1, r), dim3(kPredThreads),
+                                   sizeof(float) * n, st, n, act, dps, dpS, dpT, muA, u);
+            else
+                hipLaunchKernelGGL((pred_gather<false, 4>), g, dim3(kB), 0, st, n, act, dps, dpS,
+                                   dpT, muA, u);
             const unsigned *ssT = &sstart[(size_t)t * (r + 1)];
             const unsigned segBase = ssT[0], segs = ssT[r] - ssT[0];
             // in slices of at most 65,535 segments (the grid's y extent)

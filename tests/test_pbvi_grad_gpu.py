@@ -102,3 +102,43 @@ def test_replay_full_size_vs_fp64_replay():
     err = np.max(np.abs(dR - ref)) / np.max(np.abs(ref))
     print("PBVI replay n=5000: max |dR - dR_fp64| / max|dR_fp64| = %.3g" % err)
     assert err <= 1e-4
+
+
+@pytest.mark.parametrize("n,r,ns", [(36_864, 256, 2), (36_865, 256, 2),    # mu fits LDS, or not
+                                    (36_864, 3, 2), (300, 255, 5), (300, 256, 5), (1, 256, 1)])
+def test_replay_at_the_limits_of_the_predecessor_gather(n, r, ns):
+    """mu in LDS (at least 256 alphas of at most 36,864 states) and mu gathered from L2, with one
+    state that has a long predecessor list and rows that end early, against the FP64 replay."""
+    P = synth.pomdp_arrays(n=n, m=3, z=2, ns=ns, r=r, rz=min(n, 4), seed=n + r, gamma=0.9,
+                           horizon=3)
+    P["S"] = P["S"].copy()
+    P["S"][: n // 2, 0, 0] = 0
+    P["S"][n // 2:, 1, -1] = -1
+    res = pbvi_objective(P, P["R"])
+    dR = pbvi_replay_grad(res).cpu().numpy()
+    z = P["O"].shape[2]
+    ref = numpy_replay(P, res["recJ"].cpu().numpy().reshape(3, r, z),
+                       res["recA"].cpu().numpy().reshape(3, r), res["arg"].cpu().numpy())
+    assert np.max(np.abs(dR - ref)) <= 1e-4 * np.max(np.abs(ref))
+
+
+def test_replay_of_few_alphas_spreads_over_the_states():
+    """A step of a replay of 8 alphas of 100,000 states (26 MB of lists and rows) takes well below
+    half a millisecond; with one workgroup per alpha it takes more than one."""
+    import time
+    times = {}
+    for horizon in (4, 44):
+        P = synth.pomdp_arrays(n=100_000, m=4, z=4, ns=8, r=8, rz=8, seed=1, gamma=0.95,
+                               horizon=horizon)
+        res = pbvi_objective(P, P["R"])
+        best = np.inf
+        for _ in range(5):
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            pbvi_replay_grad(res)
+            torch.cuda.synchronize()
+            best = min(best, time.perf_counter() - t)
+        times[horizon] = best
+    step = (times[44] - times[4]) / 40
+    print("replay step, r = 8, n = 100,000: %.0f us" % (step * 1e6))
+    assert step <= 5e-4
