@@ -1870,10 +1870,15 @@ struct FusedSupport {
 
 // Words of a group: 4 (kEnd, uEnd, its value, pad), sK, bK, startK, counts, the pairs, scores,
 // alpha and j*
+// Whether the alpha's inner sums run in parallel over (observation, state): where a group has two
+// lanes and more per state.
+__host__ __device__ inline bool fused_split(unsigned n, unsigned z)
+{
+    return 2 * n <= (unsigned)kPB && z * n <= (unsigned)kFS;
+}
 __host__ __device__ inline unsigned fused_score_words(unsigned n, unsigned z, unsigned r)
 {
-    const unsigned inner = z * n <= (unsigned)kFS ? z * n : 0u;
-    return max(z * r, inner);
+    return max(z * r, fused_split(n, z) ? z * n : 0u);
 }
 __host__ __device__ inline unsigned fused_group_words(unsigned n, unsigned ns, unsigned z,
                                                       unsigned r, unsigned rz)
@@ -1883,12 +1888,15 @@ __host__ __device__ inline unsigned fused_group_words(unsigned n, unsigned ns, u
 
 // The scores of every (observation, alpha): lane t takes alpha t mod jl (jl a power of two) and Q
 // observations at a time, kPB / jl apart, so one read of Gamma serves Q sums. The support's
-// pairs are the same for every lane; four of them are read together, then their Gamma and O*T
-// values, then their sums follow in the reference's order. At one wave per SIMD the chains of
-// LDS reads were the iteration's time: with them and the actions one after another, nova's CPU
-// case (n = 64, m = 4, z = 8, ns = 4, r = 128, rz = 8) took 84.5 us an iteration; with batched
-// reads (here and for the alpha's inner sums) 39.9 us, with four actions side by side 19.0 us.
-template <int Q>
+// pairs are the same for every lane; E of them (four, or one where
+// every list has one successor: repeats of it would take LDS reads; n = 64, m = 1, z = 3, ns = 1, r = 14, rz = 60: 27 us an iteration
+// in fours, 21 one by one) are read together, then their Gamma and O*T values, then their sums
+// follow in the reference's order. At one wave per SIMD the chains of LDS reads were the
+// iteration's time: with them and the actions one after another, nova's CPU case (n = 64, m = 4,
+// z = 8, ns = 4, r = 128, rz = 8) took 84.5 us an iteration; with batched reads (here and for the
+// alpha's inner sums) 39.9 us, with four actions side by side 19.0 us. A model with one action
+// gains nothing from the latter; its iterations take up to a tenth longer than without the groups.
+template <int Q, int E>
 __device__ __forceinline__ void fused_scores(const FusedSupport &L, const float *ota,
         const float *G, float *sc, unsigned n, unsigned ns, unsigned z, unsigned r, unsigned gs,
         unsigned jl, float gamma, unsigned t)
@@ -1914,23 +1922,23 @@ __device__ __forceinline__ void fused_scores(const FusedSupport &L, const float 
 #pragma unroll
                 for (int q = 0; q < Q; q++)
                     vt[q] = 0.0f;
-                for (int u0 = first; u0 < u1; u0 += 4) {
-                    int sp[4], ou[4];
+                for (int u0 = first; u0 < u1; u0 += E) {
+                    int sp[E], ou[E];
 #pragma unroll
-                    for (int e = 0; e < 4; e++) {
+                    for (int e = 0; e < E; e++) {
                         sp[e] = L.spU[min(u0 + e, u1 - 1)];
                         ou[e] = L.otU[min(u0 + e, u1 - 1)];
                     }
-                    float g[4], w[Q][4];
+                    float g[E], w[Q][E];
 #pragma unroll
-                    for (int e = 0; e < 4; e++) {
+                    for (int e = 0; e < E; e++) {
                         g[e] = Gj[sp[e]];
 #pragma unroll
                         for (int q = 0; q < Q; q++)
                             w[q][e] = ot[q][ou[e]];
                     }
 #pragma unroll
-                    for (int e = 0; e < 4; e++)
+                    for (int e = 0; e < E; e++)
                         if (u0 + e < u1) {
 #pragma unroll
                             for (int q = 0; q < Q; q++)
@@ -1949,6 +1957,7 @@ __device__ __forceinline__ void fused_scores(const FusedSupport &L, const float 
     }
 }
 
+template <int E>
 __global__ __launch_bounds__(kFGroups * kPB) void pbvi_fused(const PbviInst *__restrict__ insts,
         const unsigned *__restrict__ off, unsigned count, unsigned iter, unsigned flip)
 {
@@ -2019,9 +2028,9 @@ __global__ __launch_bounds__(kFGroups * kPB) void pbvi_fused(const PbviInst *__r
     float bestValue = kLow;            // the same in every lane
     int bestA = -1;
     for (unsigned a0 = 0; a0 < m; a0 += groups) {
-        // the round's actions side by side; a group without one repeats the last action (its
-        // lanes keep the barriers whole, its writes repeat that action's) and is left out of the
-        // choice below
+        // the round's actions side by side; a group without one only keeps the barriers whole
+        // (its work would take LDS reads from the others) and is left out of the choice below
+        const bool idle = a0 + group >= m;
         const unsigned a = min(a0 + group, m - 1);
         const float *ota = OTall + (size_t)a * zn;
         const int *Sa = Sall + (size_t)a * sn;
@@ -2031,21 +2040,21 @@ __global__ __launch_bounds__(kFGroups * kPB) void pbvi_fused(const PbviInst *__r
         build_support(L, 0, 0, 1, ns, rz, Sa, Zi, Bi, scratch, t);   // ends with a barrier
         const int kEnd = L.kEnd;
         // score of alpha j under observation o: sum_k ((sum_l (O*T) * Gamma[j, sp]) * gamma) * b_k
-        {
+        if (!idle) {
             const unsigned jl = min((unsigned)kPB, 1u << (32 - __clz((int)max(r, 2u) - 1)));
             const unsigned across = kPB / jl;
             if (z <= across)
-                fused_scores<1>(L, ota, G, sc, n, ns, z, r, gs, jl, gamma, t);
+                fused_scores<1, E>(L, ota, G, sc, n, ns, z, r, gs, jl, gamma, t);
             else if (z <= 2 * across)
-                fused_scores<2>(L, ota, G, sc, n, ns, z, r, gs, jl, gamma, t);
+                fused_scores<2, E>(L, ota, G, sc, n, ns, z, r, gs, jl, gamma, t);
             else
-                fused_scores<4>(L, ota, G, sc, n, ns, z, r, gs, jl, gamma, t);
+                fused_scores<4, E>(L, ota, G, sc, n, ns, z, r, gs, jl, gamma, t);
         }
         __syncthreads();
         // first maximiser per observation by strict '>' from -1e10 (none: alpha 0): 32 lanes
         // per observation scan the alphas j = l, l + 32, ... in order, then merge by (value,
         // lower j)
-        for (unsigned o0 = 0; o0 < z; o0 += kPB / 32) {
+        for (unsigned o0 = idle ? z : 0; o0 < z; o0 += kPB / 32) {
             const unsigned o = o0 + t / 32, l = t % 32;
             float best = kLow;
             int bj = INT_MAX;
@@ -2079,33 +2088,33 @@ __global__ __launch_bounds__(kFGroups * kPB) void pbvi_fused(const PbviInst *__r
             const float *ot = ota + ((size_t)o * n + s) * ns;
             float vt = 0.0f;
             bool end = false;
-            for (unsigned l0 = 0; l0 < ns && !end; l0 += 4) {
-                int sp[4];
-                float w[4], g[4];
+            for (unsigned l0 = 0; l0 < ns && !end; l0 += E) {
+                int sp[E];
+                float w[E], g[E];
 #pragma unroll
-                for (unsigned e = 0; e < 4; e++) {
+                for (int e = 0; e < E; e++) {
                     const unsigned l = min(l0 + e, ns - 1);
                     sp[e] = rw[l];
                     w[e] = ot[l];
                 }
 #pragma unroll
-                for (unsigned e = 0; e < 4; e++)
+                for (int e = 0; e < E; e++)
                     g[e] = Gj[max(sp[e], 0)];
 #pragma unroll
-                for (unsigned e = 0; e < 4; e++) {
+                for (int e = 0; e < E; e++) {
                     end = end || l0 + e >= ns || sp[e] < 0;
                     vt = end ? vt : __fadd_rn(vt, __fmul_rn(w[e], g[e]));
                 }
             }
             return __fmul_rn(vt, gamma);
         };
-        const bool split = z * n <= (unsigned)kFS;
+        const bool split = fused_split(n, z);
         if (split) {
-            for (unsigned x = t; x < z * n; x += kPB)
+            for (unsigned x = idle ? z * n : t; x < z * n; x += kPB)
                 sc[x] = inner(x / n, x % n);
             __syncthreads();
         }
-        for (unsigned s = t; s < n; s += kPB) {
+        for (unsigned s = idle ? n : t; s < n; s += kPB) {
             float al = Rall[(size_t)s * m + a];
             if (split) {
 #pragma unroll 8
@@ -2118,7 +2127,7 @@ __global__ __launch_bounds__(kFGroups * kPB) void pbvi_fused(const PbviInst *__r
             alpha[s] = al;
         }
         __syncthreads();
-        if (t < 64) {
+        if (t < 64 && !idle) {
             // the products of 64 support entries at a time, then their sum in order
             float v = 0.0f;
             for (int k0 = 0; k0 < kEnd; k0 += 64) {
@@ -2495,6 +2504,8 @@ static int fused_fits(const PbviInst &I, int mode)
     return groups;
 }
 
+typedef void (*FusedFn)(const PbviInst *, const unsigned *, unsigned, unsigned, unsigned);
+
 // A launch plan over a set of instances: device descriptors and per-stage offsets.
 struct DenseWs;
 
@@ -2510,6 +2521,7 @@ struct PbviPlan {
     unsigned totTr = 0, totSc[kVariants] = {}, totBe = 0, totFu = 0;
     size_t fuLds = 0;                // dynamic LDS of pbvi_fused: the largest fused instance's
     int fuGroups = 0;                // its action groups, the same for every fused instance
+    FusedFn fuKernel = pbvi_fused<4>;
     size_t ldsBytes = 0;             // dynamic LDS of pbvi_materialize, fast and exact
     size_t ldsExact = 0;
     size_t actLds = 2 * sizeof(float) * kKMax;   // dynamic LDS of pbvi_action
@@ -2574,9 +2586,13 @@ static int plan_upload(PbviPlan &pl, void *dst, hipStream_t st, const char *fn)
     pl.maxHorizon = 0;
     // one launch has one width: every fused instance runs with the fewest groups among them
     pl.fuGroups = 0;
+    pl.fuKernel = pbvi_fused<1>;
     for (const PbviInst &I : pl.host)
-        if (I.fused)
+        if (I.fused) {
             pl.fuGroups = pl.fuGroups ? std::min(pl.fuGroups, I.fused) : I.fused;
+            if (I.ns > 1)
+                pl.fuKernel = pbvi_fused<4>;
+        }
     for (unsigned b = 0; b < c; b++) {
         PbviInst &I = pl.host[b];
         if (I.fused)
@@ -2615,7 +2631,7 @@ static int plan_upload(PbviPlan &pl, void *dst, hipStream_t st, const char *fn)
         ea = hipFuncSetAttribute((const void *)pbvi_action<false>,
                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl.actLds);
     if (ea == hipSuccess && pl.totFu > 0)
-        ea = hipFuncSetAttribute((const void *)pbvi_fused,
+        ea = hipFuncSetAttribute((const void *)pl.fuKernel,
                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)kFLds);
     if (ea != hipSuccess)
         return hip_fail(ea, fn, "Failed to set up the one-launch PBVI kernel.",
@@ -2745,7 +2761,7 @@ static void plan_enqueue(const PbviPlan &pl, unsigned iter, unsigned flip, int m
     const unsigned *tr = pl.dOff, *be = pl.dOff + (kVariants + 1) * (c + 1);
     const unsigned *fu = pl.dOff + (kVariants + 2) * (c + 1);
     if (pl.totFu > 0)
-        hipLaunchKernelGGL(pbvi_fused, dim3(pl.totFu), dim3(kPB * pl.fuGroups), pl.fuLds, st, pl.dInst, fu, c,
+        hipLaunchKernelGGL(pl.fuKernel, dim3(pl.totFu), dim3(kPB * pl.fuGroups), pl.fuLds, st, pl.dInst, fu, c,
                            iter, flip);
     if (pl.totBe == 0)
         return;
@@ -3564,7 +3580,7 @@ int pomdp_pbvi_profile_gpu(const POMDP *pomdp, POMDPPBVIGPU *pbvi, float *stageM
         // a small instance: the whole iteration is one launch, reported as the score stage
         hipEventRecord(ev[0], st);
         hipEventRecord(ev[1], st);
-        hipLaunchKernelGGL(pbvi_fused, dim3(pl.totFu), dim3(kPB * pl.fuGroups), pl.fuLds, st, pl.dInst,
+        hipLaunchKernelGGL(pl.fuKernel, dim3(pl.totFu), dim3(kPB * pl.fuGroups), pl.fuLds, st, pl.dInst,
                            pl.dOff + (kVariants + 2) * (c + 1), c, 0u, flip);
         hipEventRecord(ev[2], st);
         hipEventRecord(ev[3], st);

@@ -113,6 +113,8 @@ def test_exact_fused_equals_four_kernels_and_oracle(oracle, monkeypatch, name):
 @pytest.mark.parametrize("n,m,z,ns,r,rz", [
     (40, 2, 3, 3, 20, 5), (30, 3, 17, 4, 15, 30), (33, 5, 4, 5, 300, 12), (90, 7, 2, 2, 9, 80),
     (64, 4, 1, 8, 256, 1), (20, 8, 40, 3, 33, 7),
+    # one successor and two; states at the limit of the parallel inner sums (128); one action
+    (128, 5, 2, 1, 30, 6), (129, 3, 9, 2, 17, 9), (300, 2, 4, 1, 10, 3), (60, 1, 3, 1, 14, 60),
 ])
 def test_action_groups_equal_four_kernels(monkeypatch, n, m, z, ns, r, rz):
     """Two or four actions of a belief side by side: rounds that are not full, supports above and
@@ -124,6 +126,24 @@ def test_action_groups_equal_four_kernels(monkeypatch, n, m, z, ns, r, rz):
     for t, (a, b) in enumerate(zip(fused, updates(P, EXACT, 4))):
         assert np.array_equal(bits(a[0]), bits(b[0])), t
         assert all(np.array_equal(x, y) for x, y in zip(a[1:], b[1:])), t
+
+
+def test_iterations_of_short_lists_and_idle_groups_keep_their_time():
+    """Lists of one successor must not cost what lists of four do, and five actions (two rounds of
+    four groups, three of them without an action) not what eight do."""
+    def us(m, ns):
+        P = synth.pomdp_arrays(n=64, m=m, z=3, ns=ns, r=60, rz=60, seed=1, gamma=0.95, horizon=1)
+        set_mode(FAST)
+        p = POMDP.from_dict(P)
+        p.initialize_gpu()
+        s = POMDPPBVIGPU(p, GammaInitial=P["Gamma0"])
+        return min(s.run(20) for _ in range(12)) / 20 * 1e3
+
+    one, four, five, eight = us(1, 1), us(1, 4), us(5, 4), us(8, 4)
+    print("us an iteration: ns = 1 %.1f, ns = 4 %.1f; m = 5 %.1f, m = 8 %.1f"
+          % (one, four, five, eight))
+    assert one <= 0.8 * four
+    assert five <= 0.9 * eight
 
 
 @pytest.mark.parametrize("name", ["tiny", "mid", "n_above_block"])
