@@ -13,7 +13,8 @@ namespace nova {
 
 // Runs `sweeps` Bellman sweeps on the device continuing from vi's state (the V/VPrime
 // ping-pong by parity of currentHorizon, exactly as `sweeps` calls of mdp_vi_update_gpu), as
-// one captured HIP graph on the library stream, then synchronises. When d_V0 is non-null it
+// one captured HIP graph on the library stream, or in one launch where the model fits one
+// workgroup's LDS and sweeps >= 2, then synchronises. When d_V0 is non-null it
 // is first copied (device to device, n floats) into d_V and d_VPrime and currentHorizon is
 // reset to 0. elapsedMs (nullable) receives the device time of the sweeps alone, measured
 // with HIP events on the stream the sweeps run on.
@@ -22,11 +23,13 @@ extern "C" int mdp_vi_run_gpu(const MDP *mdp, MDPVIGPU *vi, const float *d_V0,
 
 // ---- differentiable value iteration
 
-// Which sweep kernel a solver runs: 0 = one thread per state, 1 = the wave-tiled sweep,
+// Which kernel a solver's single sweep runs: 0 = one thread per state, 1 = the wave-tiled sweep,
 // 2 = the successor-sorted tiles, 3 = the successor-chunked passes (V chunks in LDS, products
 // through HBM) that mdp_vi_initialize_gpu lays out for models of at least 2^24 (state, action,
 // successor) slots with ns <= 255 (NOVA_AMD_VI_KERNEL=tiled|sorted|chunked overrides the size
-// rule where the shape allows). All of them give the same V and pi bit for bit.
+// rule where the shape allows). Where it is 0 or 1, runs of two sweeps or more of a model that
+// fits one workgroup's LDS take one launch for all sweeps instead (NOVA_AMD_VI_KERNEL=tiled keeps
+// the launch per sweep). All of them give the same V and pi bit for bit.
 extern "C" int mdp_vi_sweep_kernel_gpu(const MDP *mdp, const MDPVIGPU *vi, unsigned int *kernel);
 
 // Batched value iteration (no counterpart in the reference): solves count MDPs (each resident

@@ -553,8 +553,8 @@ __global__ __launch_bounds__(kGThreads) void dense_score_bf16(unsigned rows, uns
 // the smaller here at every size measured (values within +-3): n = 50: 4.1e-8 against 1.1e-7,
 // n = 256: 7.9e-8 against 2.3e-7, n = 3,000: 3.0e-7 against 8.3e-7, n = 20,000: 7.5e-7 against
 // 2.1e-6 (7.8e-7 against 2.2e-6 around -20); a row of one nonzero is the exception, 3.3e-8
-// against 2.5e-8. k = 16,384, r = 4,096, n = 20,000: 20.7 -> 12.4 ms a call, the GEMM 11.6 ms:
-// 1.39 PFLOP/s of bf16 products, 0.55 of the peak (0.50 of it in dense_score_bf16, whose LDS
+// against 2.5e-8. k = 16,384, r = 4,096, n = 20,000: 20.9 -> 13.0 ms a call, the GEMM 12.2 ms:
+// 1.32 PFLOP/s of bf16 products, 0.53 of the peak (0.50 of it in dense_score_bf16, whose LDS
 // reads per matrix instruction are half as many again).
 //
 // Operands lie in the order in which lanes read them from LDS: 1 KB blocks of 32 rows x 16 k,
@@ -626,7 +626,8 @@ __global__ __launch_bounds__(kGConvThreads) void dense_split_convert(unsigned n,
 // roundings, the fp32 instruction one (rms relative error at n = 1,000, rows of 64 nonzeros:
 // 2.3e-7 in one pass, 4.3e-8 in two, 1.2e-7 with the fp32 instruction; dense rows at n = 20,000:
 // 1.7e-6 and 7.5e-7). The second pass copies a third of the bytes once more: k = 16,384,
-// r = 4,096, n = 20,000: 11.9 -> 12.4 ms a call.
+// r = 4,096, n = 20,000: 12.6 -> 13.0 ms a call. (256 x 128 tiles with sums of their own for the hh
+// products copy half the bytes once more, and the copies past L2 are what bounds it: 15.8 ms.)
 __global__ __launch_bounds__(kGThreads) void dense_score_split(unsigned rows, unsigned cols,
         unsigned kpad, unsigned rowTiles, unsigned colTiles, const __bf16 *__restrict__ A,
         const __bf16 *__restrict__ B, float *__restrict__ partVal, int *__restrict__ partJ,

@@ -15,7 +15,10 @@
 //   * row sums are staged in LDS; one lane per state then takes the max over actions with the
 //     reference's tie rule, and V'/pi are written coalesced.
 // A plain one-thread-per-state kernel covers shapes the tiled kernel does not (ns > 256,
-// m > 2048, misaligned arrays).
+// m > 2048, misaligned arrays). Runs of several sweeps of a model that fits one workgroup's LDS
+// take one launch (vi_resident); large models get a layout of their own at initialize
+// (successor-sorted tiles, successor chunks); batches of models share a launch per sweep
+// (vi_batch_sweep).
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>

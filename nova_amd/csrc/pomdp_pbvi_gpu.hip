@@ -1888,8 +1888,8 @@ __host__ __device__ inline unsigned fused_group_words(unsigned n, unsigned ns, u
 
 // The scores of every (observation, alpha): lane t takes alpha t mod jl (jl a power of two) and Q
 // observations at a time, kPB / jl apart, so one read of Gamma serves Q sums. The support's
-// pairs are the same for every lane; E of them (four, or one where
-// every list has one successor: repeats of it would take LDS reads; n = 64, m = 1, z = 3, ns = 1, r = 14, rz = 60: 27 us an iteration
+// pairs are the same for every lane; E of them (four, or one where every list has one successor:
+// repeats of it would take LDS reads; n = 64, m = 1, z = 3, ns = 1, r = rz = 60: 27 us an iteration
 // in fours, 21 one by one) are read together, then their Gamma and O*T values, then their sums
 // follow in the reference's order. At one wave per SIMD the chains of LDS reads were the
 // iteration's time: with them and the actions one after another, nova's CPU case (n = 64, m = 4,
@@ -2761,8 +2761,8 @@ static void plan_enqueue(const PbviPlan &pl, unsigned iter, unsigned flip, int m
     const unsigned *tr = pl.dOff, *be = pl.dOff + (kVariants + 1) * (c + 1);
     const unsigned *fu = pl.dOff + (kVariants + 2) * (c + 1);
     if (pl.totFu > 0)
-        hipLaunchKernelGGL(pl.fuKernel, dim3(pl.totFu), dim3(kPB * pl.fuGroups), pl.fuLds, st, pl.dInst, fu, c,
-                           iter, flip);
+        hipLaunchKernelGGL(pl.fuKernel, dim3(pl.totFu), dim3(kPB * pl.fuGroups), pl.fuLds, st,
+                           pl.dInst, fu, c, iter, flip);
     if (pl.totBe == 0)
         return;
     hipLaunchKernelGGL(pbvi_transpose, dim3(pl.totTr), dim3(kPB), 0, st, pl.dInst, tr, c, iter, flip);
@@ -3580,8 +3580,8 @@ int pomdp_pbvi_profile_gpu(const POMDP *pomdp, POMDPPBVIGPU *pbvi, float *stageM
         // a small instance: the whole iteration is one launch, reported as the score stage
         hipEventRecord(ev[0], st);
         hipEventRecord(ev[1], st);
-        hipLaunchKernelGGL(pl.fuKernel, dim3(pl.totFu), dim3(kPB * pl.fuGroups), pl.fuLds, st, pl.dInst,
-                           pl.dOff + (kVariants + 2) * (c + 1), c, 0u, flip);
+        hipLaunchKernelGGL(pl.fuKernel, dim3(pl.totFu), dim3(kPB * pl.fuGroups), pl.fuLds, st,
+                           pl.dInst, pl.dOff + (kVariants + 2) * (c + 1), c, 0u, flip);
         hipEventRecord(ev[2], st);
         hipEventRecord(ev[3], st);
         hipEventRecord(ev[4], st);

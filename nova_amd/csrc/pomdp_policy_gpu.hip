@@ -21,11 +21,13 @@
 //    sum_s T[s,a,s'] b(s), normalised by its sum over s'. The sum over predecessors runs over a
 //    list ordered by (s, successor slot) -- the order in which the reference's scatter adds to
 //    b'(s') -- and the normaliser is summed serially over s' ascending, so b' equals nova's
-//    bit for bit. Three kernels: the unnormalised b' (predecessor entries read coalesced, their
-//    products summed per s' from LDS, b gathered from LDS, O from an observation-major copy
-//    built once per model), the normalisers (one serial chain per triple fed through LDS), and
-//    the division. A triple whose normaliser is below 1e-9 in magnitude keeps the unnormalised
-//    b' and reports NOVA_WARNING_INVALID_BELIEF, as the reference returns it.
+//    bit for bit. Three kernels, four where many triples are tiled (belief_tiles lays their
+//    beliefs out, belief_update_tiles forms 32 b' per list entry read): the unnormalised b'
+//    (predecessor entries read coalesced, their products summed per s' from LDS, b gathered from
+//    LDS, O from an observation-major copy built once per model), the normalisers (one serial
+//    chain per triple fed through LDS), and the division. A triple whose normaliser is below
+//    1e-9 in magnitude keeps the unnormalised b' and reports NOVA_WARNING_INVALID_BELIEF, as the
+//    reference returns it.
 #include <algorithm>
 #include <climits>
 #include <cstdint>
@@ -389,9 +391,9 @@ void launch_few_of(unsigned few, unsigned k, unsigned n, unsigned r, const float
 // 315 / 177 / 82). bf16 calls take it up to kFewBf16 beliefs (n = 20,000, r = 4,096: k = 8: 213,
 // k = 64: 408 against 508 of the bf16 GEMM at any k up to 256).
 // Short rows leave nothing to spread: exact calls of at most kFewShort states, and of many
-// pairs (kFewShortPairs) in both directions, keep the square tiles (n = 50: k = 1,000, r = 1,200: 34 / 34;
-// k = 18,750, r = 64: 29 / 34; k = 50,000, r = 20: 34 / 38; k = 9,375, r = 64: 29 / 28;
-// k = 75,000, r = 16: 40 / 34; n = 100: k = 18,750, r = 64: 38 / 34).
+// pairs (kFewShortPairs) in both directions, keep the square tiles (n = 50: k = 1,000,
+// r = 1,200: 34 / 34; k = 18,750, r = 64: 29 / 34; k = 50,000, r = 20: 34 / 38; k = 9,375, r = 64:
+// 29 / 28; k = 75,000, r = 16: 40 / 34; n = 100: k = 18,750, r = 64: 38 / 34).
 // The partials of k >= kMergeWaves beliefs (at most 10 tiles each) are merged a lane per belief,
 // fewer a wave per belief (us of a call, wave / lane: n = 50, k = 50,000, r = 20: 49 / 38;
 // k = 8,192, r = 10: 24 / 22; k = 4,096, r = 300: 36 / 40).
@@ -644,9 +646,9 @@ constexpr size_t kTileBytes = (size_t)128 << 20;     // most state-major beliefs
 
 template <typename IDX>
 __global__ __launch_bounds__(kTileThreads) void belief_update_tiles(unsigned n, unsigned z,
-        unsigned blocks, unsigned count, unsigned spread, const uint4 *__restrict__ tiles, const unsigned *__restrict__ order,
-        const unsigned *__restrict__ pstart, const IDX *__restrict__ pS,
-        const float *__restrict__ pT, const float *__restrict__ O,
+        unsigned blocks, unsigned count, unsigned spread, const uint4 *__restrict__ tiles,
+        const unsigned *__restrict__ order, const unsigned *__restrict__ pstart,
+        const IDX *__restrict__ pS, const float *__restrict__ pT, const float *__restrict__ O,
         const unsigned *__restrict__ obs, const float *__restrict__ BT, float *__restrict__ Bp)
 {
     __shared__ float buf[kTileT][kTileS + 1];

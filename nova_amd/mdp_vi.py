@@ -86,7 +86,8 @@ class MDPValueIterationGPU(_abi.NovaMDPVIGPU):
         return policy
 
     def run(self, sweeps, d_V0=None):
-        """Runs `sweeps` sweeps on the device (one graph); returns their device time in ms.
+        """Runs `sweeps` sweeps on the device (one graph, or one launch where the model fits a
+        workgroup's LDS); returns their device time in ms.
         d_V0: optional device pointer (int) of n floats to restart from."""
         ms = ct.c_float(0.0)
         rc = self._lib.mdp_vi_run_gpu(self.mdpPtr, self, d_V0, sweeps, ct.byref(ms))
@@ -95,8 +96,10 @@ class MDPValueIterationGPU(_abi.NovaMDPVIGPU):
         return ms.value
 
     def sweep_kernel(self):
-        """0: one thread per state, 1: wave-tiled sweep, 2: successor-sorted tiles,
-        3: successor chunks (V chunks in LDS, products through HBM)."""
+        """The kernel of a single sweep. 0: one thread per state, 1: wave-tiled sweep,
+        2: successor-sorted tiles, 3: successor chunks (V chunks in LDS, products through HBM).
+        Where it is 0 or 1, runs of two sweeps or more of a model that fits one workgroup's LDS
+        take one launch for all sweeps instead."""
         k = ct.c_uint(0)
         if self._lib.mdp_vi_sweep_kernel_gpu(self.mdpPtr, self, ct.byref(k)) != 0:
             raise Exception("mdp_vi_sweep_kernel_gpu failed")

@@ -3,9 +3,11 @@ oracle: nova_amd_alpha_vectors_value_and_action_gpu (pomdp_alpha_vectors.cpp:52-
 and nova_amd_belief_update_batch_gpu (pomdp_model_cpu.cpp:89-137 per triple).
 
 exact value/action and the belief update: bit for bit against the oracle's float twin.
-fp32 (matrix cores): the chosen alpha is the FP64 maximiser except at near-ties (its FP64
+Calls of at most 1.25 Mi (belief, alpha) pairs (exact ones of short rows: 576 Ki; bf16: at most 64
+beliefs) run on the vector ALUs, one wave per 16 alphas; the sizes below lie on both sides.
+fp32: the chosen alpha is the FP64 maximiser except at near-ties (its FP64
       value within 1e-5 * max(1, |V|) of the maximum) and V within 1e-5 relative.
-bf16 (matrix cores): reported (alpha disagreement rate, value error against FP64); the value
+bf16: reported (alpha disagreement rate, value error against FP64); the value
       of the chosen alpha stays within 1e-2 * max |V| of the FP64 maximum.
 """
 import ctypes as ct
@@ -177,7 +179,8 @@ def test_exact_no_alpha_above_sentinel():
         assert np.all(act.cpu().numpy() == 0) and np.all(j.cpu().numpy() == -1), prec
 
 
-@pytest.mark.parametrize("k,n,r", SHAPES[1:] + [(4096, 2000, 1024)])
+# the last two on the matrix cores, the others below their 1.25 Mi pairs
+@pytest.mark.parametrize("k,n,r", SHAPES[1:] + [(2100, 257, 700), (4096, 2000, 1024)])
 def test_fp32_matrix_cores_vs_fp64(k, n, r):
     G, pi, B = instance(k, n, r, seed=3 * k + r)
     p = policy(G, pi)
@@ -291,6 +294,21 @@ def test_fp32_operands_without_bf16_parts(odd):
     assert np.allclose(V[fine], best[fine], rtol=1e-5, atol=1e-5)
     assert np.array_equal(V[~fine], best[~fine])
     assert np.all(j[~fine] == 11)
+
+
+@pytest.mark.parametrize("k,n,r", [(1400, 513, 1000), (1024, 600, 1300), (700, 1000, 2000)])
+def test_fp32_fallback_vs_fp64(k, n, r):
+    """The fp32 matrix instructions, which take the calls whose operands have no bf16 parts, over rows
+    of many steps, full and ragged: V within n fp32 roundings of the FP64 maximum."""
+    G, pi, B = instance(k, n, r, seed=k + n)
+    B[0, 0] = 1e-36
+    V, act, j = policy(G, pi).value_and_action_batch(B, "fp32", return_alpha=True)
+    V, act, j = V.cpu().numpy(), act.cpu().numpy(), j.cpu().numpy()
+    C = B.astype(np.float64) @ G.astype(np.float64).T
+    bound = (n + 1) * 2.0 ** -24 * (np.abs(B).astype(np.float64) @ np.abs(G).T).max(axis=1)
+    assert np.all(np.abs(V - C.max(axis=1)) <= bound)
+    assert np.all(C.max(axis=1) - C[np.arange(k), j] <= 2 * bound)
+    assert np.array_equal(act, pi[j])
 
 
 @pytest.mark.parametrize("x,y", [(1.998 * 2.0 ** 63, 1.9985 * 2.0 ** 63),    # just below the range

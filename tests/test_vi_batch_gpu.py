@@ -1,5 +1,5 @@
-"""Batched value iteration (mdp_vi_batch_execute_gpu): many MDPs of uneven size, every sweep
-of every instance in one HIP graph. Each instance must equal the float oracle's run
+"""Batched value iteration (mdp_vi_batch_execute_gpu): many MDPs of uneven size, one launch per
+sweep for all instances. Each instance must equal the float oracle's run
 (mdp_vi_cpu.cpp:36-63 per sweep) and its plain GPU solve bit for bit, whatever its size,
 horizon (odd, even, 1), gamma, initial values and ragged successor lists."""
 import ctypes as ct
