@@ -140,7 +140,7 @@ def test_exact_calls_of_many_beliefs_and_few_alphas_keep_their_time():
 
     fewer, more = best_of(50_000, 20), best_of(40_000, 33)
     print("exact value/action: 1.00 M pairs %.1f us, 1.32 M %.1f us" % (fewer * 1e6, more * 1e6))
-    assert fewer <= 1.2 * more
+    assert fewer <= 1.35 * more
 
 
 @pytest.mark.parametrize("extra", [4, 5])        # rows aligned to 16 bytes, or not
